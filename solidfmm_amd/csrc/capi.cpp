@@ -30,6 +30,7 @@
 
 #include "../../include/solidfmm_gpu.h"
 #include "mfma_tables.hpp"
+#include "team_tables.hpp"
 #include "translate.hpp"
 
 namespace {
@@ -261,8 +262,11 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
         rounds = std::max(rounds, round + 1);
         plan.src_extent = std::max<size_t>(plan.src_extent, it.src + size_t(it.p_in) * (it.p_in + 1));
         plan.dst_extent = std::max<size_t>(plan.dst_extent, it.dst + size_t(it.p_out) * (it.p_out + 1));
-        // the generic kernel takes every order in one launch
-        keys.push_back({round, fam, fam == sfmm::kGenericKernel ? 0u : pb, it.p_in, it.p_out, i});
+        // the generic kernels take many orders in one launch
+        uint32_t bucket = pb;
+        if (fam == sfmm::kGenericKernel)
+            bucket = ctx->precision == SFMM_FP64 ? sfmm::generic_bucket(pb) : sfmm::kGenericRest;
+        keys.push_back({round, fam, bucket, it.p_in, it.p_out, i});
     }
     plan.scratch = rounds > kMaxRounds;
     if (plan.scratch)
@@ -328,7 +332,8 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
         if (k == 0 || keys[k - 1].round != key.round || keys[k - 1].family != key.family ||
             keys[k - 1].pb != key.pb) {
             plan.launches.push_back(
-                {{key.family, key.pb, false, ctx->precision, !plan.scratch}, ordered.size(), 0, key.round});
+                {{key.family, key.family == sfmm::kGenericKernel ? 0u : key.pb, false, ctx->precision, !plan.scratch},
+                 ordered.size(), 0, key.round});
             plan.launches.back().k.seg =
                 runs && (key.family == sfmm::kLaneKernels || key.family == sfmm::kMfmaKernels);
             prev = nullptr;
@@ -544,7 +549,10 @@ hipError_t ensure_branches(sfmm_context *ctx)
 
 // Device tables the kernels read, created before any capture so that no
 // allocation happens inside one.
-bool tables_ready() { return sfmm::mfma::device_table() && sfmm::mfma::device_factorials(); }
+bool tables_ready()
+{
+    return sfmm::mfma::device_table() && sfmm::mfma::device_factorials() && sfmm::team::device_table();
+}
 
 // Device scratch of the allocation-free entry point (sfmm_translate_noalloc):
 // the plan's tables (items, reduction targets and items) and, when targets

@@ -3,8 +3,9 @@
 // translation (grid-stride over the list); the threads share the order
 // index m, the rotated triangle lives in LDS, the folded swap blocks come
 // from the dense device table (mfma_tables.hpp).  This is the complete-
-// coverage path behind the specialised kernels of translate.hip and
-// translate_mfma.hpp, which it must agree with.
+// coverage path behind the specialised kernels of lane_kernel.hpp,
+// translate_mfma.hpp and team.hpp, which it must agree with: orders above 48,
+// and lower ones where a context asks for it.
 //
 // Steps follow translations.cpp:36-471: forward transforms per input degree
 // (scale, rotate alpha, swap, rotate beta, swap), the z-translation

@@ -17,6 +17,7 @@
 
 #include "../../include/solidfmm_gpu.h"
 #include "mfma_tables.hpp"
+#include "team_tables.hpp"
 
 namespace sfmm {
 
@@ -156,6 +157,65 @@ const double *device_factorials()
 }
 
 }  // namespace mfma
+
+namespace team {
+
+namespace {
+
+// Both tables of team_tables.hpp.
+std::vector<double> build_tables()
+{
+    const SwapRecurrence &rec = recurrence();
+    std::vector<double> out(2 * size_t(table_size()), 0.0);
+    for (int n = 0; n < kMaxOrder; ++n) {
+        const int nj = chunks(n);
+        double *deg = out.data() + base_of(nj) + size_t(n - 8 * (nj - 1)) * degree_size(nj);
+        for (int block = 0; block < 4; ++block) {
+            const int part = block / 2, e = block % 2;
+            const int o = (e + n + part) & 1;  // class of the outputs
+            for (int i = 0; 2 * i + o <= n; ++i)
+                for (int j = 0; 2 * j + e <= n; ++j) {
+                    size_t at;
+                    if (nj <= kSmall) {
+                        const int p = (block * nj + i / 4) * nj + j / 4;  // operand
+                        at = size_t(p / 2) * 32 + (i % 4 + 4 * (j % 4)) * 2 + p % 2;
+                    } else {
+                        const int p = (block * row_blocks(nj) + i / 16) * nj + j / 4;
+                        at = size_t(p) * 64 + i % 16 + 16 * (j % 4);
+                    }
+                    const int m = 2 * i + o, l = 2 * j + e;
+                    deg[at] = rec.folded(n, part, m, l);
+                    deg[table_size() + at] = (l ? 2.0 : 1.0) * (m ? 0.5 : 1.0) * rec.folded(n, part, l, m);
+                }
+        }
+    }
+    return out;
+}
+
+}  // namespace
+
+const double *device_table()
+{
+    static std::mutex mu;
+    static std::vector<double *> per_device;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+    std::lock_guard<std::mutex> lock(mu);
+    if (per_device.size() <= size_t(dev)) per_device.resize(dev + 1, nullptr);
+    if (!per_device[dev]) {
+        const std::vector<double> h = build_tables();
+        double *d = nullptr;
+        if (hipMalloc(&d, h.size() * sizeof(double)) != hipSuccess) return nullptr;
+        if (hipMemcpy(d, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess) {
+            (void)hipFree(d);
+            return nullptr;
+        }
+        per_device[dev] = d;
+    }
+    return per_device[dev];
+}
+
+}  // namespace team
 }  // namespace sfmm
 
 extern "C" int sfmm_swap_block(int n, int part, double *out)

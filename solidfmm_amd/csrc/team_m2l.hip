@@ -1,0 +1,15 @@
+// Instantiations of the team kernel for M2L.
+#include "team.hpp"
+
+namespace sfmm {
+namespace team {
+
+template <>
+const Kernels &kernels<SFMM_M2L>()
+{
+    static const Kernels k{&k_team<SFMM_M2L, 4, 4, 8, 2>, &k_team<SFMM_M2L, 6, -1, 8, 2>};
+    return k;
+}
+
+}  // namespace team
+}  // namespace sfmm

@@ -2,7 +2,8 @@
 //
 // The kernels themselves live in lane_kernel.hpp (one lane per
 // translation), translate_mfma.hpp (16 translations per wave on the FP64
-// matrix cores), generic.hip (one workgroup per translation, any order) and,
+// matrix cores), team.hpp (up to 16 translations per workgroup, orders 25 to
+// 48), generic.hip (one workgroup per translation, any order) and,
 // for the reduced-precision modes, lane_prec.hpp, mfma_prec.hpp (FP32
 // matrix cores) and prec_generic.hip.
 #include <hip/hip_runtime.h>
@@ -37,6 +38,12 @@ int default_family(uint32_t pb)
     if (pb <= kLaneAutoMax) return kLaneKernels;
     if (pb <= uint32_t(mfma::kMfmaMax)) return kMfmaKernels;
     return kGenericKernel;
+}
+
+uint32_t generic_bucket(uint32_t pb)
+{
+    if (pb <= uint32_t(mfma::kMfmaMax) || pb > kTeamMax) return kGenericRest;
+    return pb <= 32 ? 32 : kTeamMax;
 }
 
 bool have_kernel(int op, uint32_t p_in, uint32_t p_out, int family)
@@ -149,7 +156,13 @@ hipError_t launch_kernel(int op, const KernelChoice &k, const sfmm_item *items, 
         return k.rt ? launch_mfma<true>(op, k.pk, items, n, src, dst, table, stream, mode)
                     : launch_mfma<false>(op, k.pk, items, n, src, dst, table, stream, mode);
     }
-    default: return launch_generic(op, k.pk, items, n, src, dst, stream, acc);
+    default:
+        // Orders above the MFMA kernels' 24 run on the team kernels as far
+        // as their LDS triangle reaches (M2L, 2,000 items: order 25 340 ->
+        // 27 us, 32 577 -> 40, 40 895 -> 84, 48 2500 -> 121; a single group
+        // of 7 items: order 32 488 -> 31).
+        if (generic_bucket(k.pk) != kGenericRest) return launch_team(op, k.pk, items, n, src, dst, stream, acc);
+        return launch_generic(op, k.pk, items, n, src, dst, stream, acc);
     }
 }
 

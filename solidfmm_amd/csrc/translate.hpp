@@ -15,8 +15,8 @@ namespace sfmm {
 //            (lane_kernel.hpp);
 //   MFMA     one wave per 16 translations, swaps on the FP64 matrix cores,
 //            orders up to 24 (translate_mfma.hpp);
-//   generic  one workgroup per translation, any orders up to 86
-//            (generic.hip).
+//   generic  any orders up to 86: 25 to 48 on the team kernels (team.hpp),
+//            the rest one workgroup per translation (generic.hip).
 // Lane and MFMA kernels are instantiated per square order PB; their RT
 // variants take items of any orders p_in, p_out <= PB.
 enum Family { kAuto = 0, kLaneKernels = 1, kMfmaKernels = 2, kGenericKernel = 3 };
@@ -68,6 +68,18 @@ hipError_t launch_prec_generic(int precision, int op, uint32_t pc, const sfmm_it
 inline constexpr uint32_t kPrecLaneAutoMax = 16;
 hipError_t launch_prec_mfma_m2l(uint32_t P, const sfmm_item *items, size_t n, const double *src, double *dst,
                                 hipStream_t stream, int acc);
+
+// Team kernels (team.hpp): items of any orders up to pc <= kTeamMax; mode as
+// there.
+inline constexpr uint32_t kTeamMax = 48;
+hipError_t launch_team(int op, uint32_t pc, const sfmm_item *items, size_t n, const double *src, double *dst,
+                       hipStream_t stream, int mode);
+
+// Launch bucket of an FP64 item of the generic family, by its larger order:
+// 32 (orders 25 to 32) and kTeamMax (33 to 48) run on team kernels of their
+// own registers and LDS, everything else together on the generic kernel.
+inline constexpr uint32_t kGenericRest = 0;
+uint32_t generic_bucket(uint32_t pb);
 
 // One launch of a plan: family (not kAuto), the kernel's order bound pk,
 // whether items carry their own orders (rt), the arithmetic (SFMM_FP64,

@@ -1,0 +1,104 @@
+"""Team kernels (several waves per group of translations) against the oracle
+-- needs an MI355X.
+
+Orders above 24 run on physical (decaying) expansions.  Error measure: per
+item, the 2-norm of the difference over the 2-norm of the oracle's block.
+Bound: 20 times the largest distance of the oracle from the naive O(P^4)
+formulas on the same items (two evaluations of one algorithm, whose errors
+sit at that distance), and not below 1e-13.
+"""
+import numpy as np
+import pytest
+
+from solidfmm_amd import workload as W
+from tests.test_gpu_translate import physical_batch
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+OPS = [W.M2M, W.M2L, W.L2L]
+
+
+@pytest.fixture(scope="module")
+def sfmm():
+    if not torch.cuda.is_available():
+        pytest.fail("GPU tests need a visible GPU")
+    import solidfmm_amd
+    solidfmm_amd.load()
+    return solidfmm_amd
+
+
+def run(sfmm, op, items, src, dst0, family=0):
+    ctx = sfmm.Context(int(max(items["p_in"].max(), items["p_out"].max())))
+    ctx.set_kernels(family)
+    plan = sfmm.Plan(ctx, op, items)
+    s, d = torch.from_numpy(src).to("cuda"), torch.from_numpy(dst0.copy()).to("cuda")
+    plan.execute(s, d)
+    torch.cuda.synchronize()
+    return d.cpu().numpy()
+
+
+def block_errors(got, want, dst0, items):
+    """Per distinct target: |got - want| / |want - dst0|."""
+    out = []
+    for off, p in sorted({(int(o), int(p)) for o, p in zip(items["dst"], items["p_out"])}):
+        sl = slice(off, off + p * (p + 1))
+        scale = np.linalg.norm(want[sl] - dst0[sl])
+        d = np.linalg.norm(got[sl] - want[sl])
+        out.append(d / scale if scale else (np.inf if d else 0.0))
+    return np.array(out)
+
+
+def check(sfmm, orc, op, items, src, dst0, label):
+    want = orc.translate(op, items, src, dst0.copy())
+    naive = orc.translate(op, items, src, dst0.copy(), naive=True)
+    tol = max(20 * block_errors(naive, want, dst0, items).max(), 1e-13)
+    err = block_errors(run(sfmm, op, items, src, dst0), want, dst0, items).max()
+    print(f"{label}: {err:.2e} (tol {tol:.2e})", flush=True)
+    assert err <= tol
+
+
+# 25 and 32: ends of the kernel with four chunks per parity class; 33: the
+# next one; 36 and 48: 8 translations per workgroup and the largest triangle
+@pytest.mark.parametrize("op", OPS)
+@pytest.mark.parametrize("P,n", [(25, 1), (25, 17), (31, 15), (32, 16), (32, 33), (33, 9), (36, 8), (36, 17),
+                                 (41, 5), (47, 9), (48, 3)])
+def test_high_orders_square(sfmm, orc, op, P, n):
+    items, src, dst = physical_batch(orc, op, P, P, n, 7 * P + n + op)
+    dst0 = 1e-3 * np.resize(src, len(dst))  # targets are added to
+    check(sfmm, orc, op, items, src, dst0, f"op {op} P={P} n={n}")
+
+
+@pytest.mark.parametrize("op", OPS)
+def test_high_orders_mixed(sfmm, orc, op):
+    """One list of order pairs up to 48 (and one above, and one below 25),
+    zero shifts among them, in shuffled order."""
+    pairs = [(25, 25), (30, 26), (26, 31), (32, 3), (2, 32), (33, 33), (48, 34), (35, 48), (1, 40), (45, 1), (50, 49),
+             (24, 20)]
+    if op == W.L2L:  # truncation beyond p_out + 1 is covered against the naive formula only
+        pairs = [(a, b) for a, b in pairs if a <= b + 1] + [(27, 26), (41, 40)]
+    rng = np.random.default_rng(11 + op)
+    parts = [physical_batch(orc, op, a, b, 5, 100 + 10 * a + b + op) for a, b in pairs]
+    so = np.cumsum([0] + [len(p[1]) for p in parts])
+    do = np.cumsum([0] + [len(p[2]) for p in parts])
+    items = []
+    for k, (it, _, _) in enumerate(parts):
+        it = it.copy()
+        it["src"] += np.uint64(so[k])
+        it["dst"] += np.uint64(do[k])
+        if op != W.M2L:
+            for c in "xyz":
+                it[c][k % 5] = 0.0
+        items.append(it)
+    items = rng.permutation(np.concatenate(items))
+    src = np.concatenate([p[1] for p in parts])
+    check(sfmm, orc, op, items, src, np.zeros(do[-1]), f"mixed op {op}")
+
+
+@pytest.mark.parametrize("P", [26, 40])
+def test_high_orders_repeated_targets(sfmm, orc, P):
+    """Targets repeated often enough for scratch blocks and a reduction."""
+    items, src, dst = physical_batch(orc, W.M2L, P, P, 29, 3 * P)
+    items["dst"] = (np.arange(29) % 4) * P * (P + 1)
+    check(sfmm, orc, W.M2L, items, src, np.zeros(len(dst)), f"repeated P={P}")
