@@ -209,17 +209,6 @@ private:
 // are applied in list order by rounds (the k-th item of a target runs in
 // launch round k); otherwise every item writes its own scratch block and a
 // segmented reduction adds a target's blocks in list order (reduce.hip).
-// Square FP64 M2L orders 21 and 22 on the MFMA kernels run faster through
-// the per-item-order variant, whose output degrees ascend with fewer
-// registers live (2e5 translations: the fixed-order kernel is 6 % slower at
-// 22, and 1-2 % faster at 18 and 20, where this choice once saved 8-14 %
-// before the swaps recomputed their indices).
-template <class K>
-bool mfma_rt_square(const K &key)
-{
-    return key.family == sfmm::kMfmaKernels && key.pb >= 21 && key.pb <= 22;
-}
-
 int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm_plan &plan)
 {
     if (op < SFMM_M2M || op > SFMM_L2L) return fail(ctx, SFMM_ERR_LOGIC, "solidfmm: unknown operator");
@@ -234,6 +223,7 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
     keys.reserve(n);
     FlatMap seen;  // target -> occurrences so far
     uint32_t rounds = 0;
+    size_t lanes[kMaxRounds][sfmm::kLaneMax + 1] = {};  // items of the lane kernels per round and order
     // kernel family per (p_in, p_out), filled on first use: lists repeat a
     // handful of order pairs millions of times
     constexpr int kNoKernel = -2, kUnknown = -1;
@@ -266,11 +256,29 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
         uint32_t bucket = pb;
         if (fam == sfmm::kGenericKernel)
             bucket = ctx->precision == SFMM_FP64 ? sfmm::generic_bucket(pb) : sfmm::kGenericRest;
+        if (fam == sfmm::kLaneKernels && pb <= sfmm::kLaneMax) ++lanes[std::min(round, kMaxRounds - 1)][pb];
         keys.push_back({round, fam, bucket, it.p_in, it.p_out, i});
     }
     plan.scratch = rounds > kMaxRounds;
     if (plan.scratch)
         for (Key &k : keys) k.round = 0;
+    // Small buckets of the lane kernels go to the MFMA family's team kernel
+    // where neither the context nor its tuning asks for lanes. Decided here,
+    // before runs are laid out by the family's wave.
+    if (ctx->precision == SFMM_FP64 && ctx->family == SFMM_KERNELS_AUTO) {
+        bool moved[kMaxRounds][sfmm::kLaneMax + 1] = {}, any = false;
+        for (uint32_t pb = 1; pb <= sfmm::kLaneMax; ++pb) {
+            if (plan.scratch)
+                for (uint32_t r = 1; r < kMaxRounds; ++r) lanes[0][pb] += lanes[r][pb];
+            for (uint32_t r = 0; r < (plan.scratch ? 1u : kMaxRounds); ++r) {
+                moved[r][pb] = lanes[r][pb] && !ctx->tune[op][pb] && lanes[r][pb] <= sfmm::lane_team_items(pb);
+                any = any || moved[r][pb];
+            }
+        }
+        if (any)
+            for (Key &k : keys)
+                if (k.family == sfmm::kLaneKernels && moved[k.round][k.pb]) k.family = sfmm::kMfmaKernels;
+    }
     // keys are in list order here: remember each item's position in it
     std::vector<uint32_t> list_pos;
     if (plan.scratch) {
@@ -341,8 +349,7 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
         sfmm_plan::Launch &L = plan.launches.back();
         if (key.family == sfmm::kGenericKernel) {
             L.k.pk = std::max({L.k.pk, key.p_in, key.p_out});
-        } else if (key.p_in != key.pb || key.p_out != key.pb ||
-                   (op == SFMM_M2L && ctx->precision == SFMM_FP64 && mfma_rt_square(key))) {
+        } else if (key.p_in != key.pb || key.p_out != key.pb) {
             L.k.rt = true;
         }
         const sfmm_item &src_it = items[key.index];

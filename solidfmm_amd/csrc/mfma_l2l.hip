@@ -1,5 +1,5 @@
 // Instantiations of the MFMA translation kernels for L2L (square orders
-// kMfmaMin..kMfmaMax, uniform orders).
+// kMfmaMin..kMfmaKernelMax, uniform orders).
 #include "translate_mfma.hpp"
 
 namespace sfmm {

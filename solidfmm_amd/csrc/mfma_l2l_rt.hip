@@ -1,5 +1,5 @@
 // Instantiations of the MFMA translation kernels for L2L (square orders
-// kMfmaMin..kMfmaMax, runtime per-item orders).
+// kMfmaMin..kMfmaKernelMax, runtime per-item orders).
 #include "translate_mfma.hpp"
 
 namespace sfmm {

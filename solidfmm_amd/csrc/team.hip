@@ -45,15 +45,23 @@ hipError_t launch_team(int op, uint32_t pc, const sfmm_item *items, size_t n, co
     const Kernels &ks = op == SFMM_M2M   ? kernels<SFMM_M2M>()
                         : op == SFMM_M2L ? kernels<SFMM_M2L>()
                                          : kernels<SFMM_L2L>();
-    const int njx = pc > 32 ? 6 : 4;
+    const int njx = pc > 32 ? 6 : pc > 24 ? 4 : pc > 16 ? 3 : 2;
     // as many translations as the triangle leaves room for: 16 up to order
     // 32 (fixed in that kernel), 8 up to 48
     int tl = 4;
     while (lds_bytes(op, njx, int(pc), tl) > kLds) --tl;
     const size_t lds = lds_bytes(op, njx, int(pc), tl);
     const size_t groups = (n + (size_t(1) << tl) - 1) >> tl;
-    const int waves = 8;  // one workgroup per CU: its LDS is taken
-    const fn_t f = njx == 6 ? ks.upto48 : ks.upto32;
+    // Eight waves while every group has a CU of its own (the shortest chain
+    // of degrees a wave), four beyond: two or three groups share a CU and one
+    // group's waits for memory and barriers cover another's (order 16, 4,000
+    // items: 14 us with eight waves, 16 with four; 8,000: 24 and 22; 24,000:
+    // 60 and 52).
+    const int waves = pc > 24 || groups <= 256 ? 8 : 4;
+    const fn_t f = njx == 6   ? ks.upto48
+                   : njx == 4 ? ks.upto32
+                   : njx == 3 ? (waves == 8 ? ks.upto24w : ks.upto24)
+                             : (waves == 8 ? ks.upto16w : ks.upto16);
     if (lds > 64 * 1024) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(f),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, int(kLds));

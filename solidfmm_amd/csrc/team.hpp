@@ -28,6 +28,9 @@
 // vector instructions share.  M2L of order 32: 2,003 translations 577 us on
 // the one-workgroup-per-translation kernel, 37 us here; 30,000 7.7 ms and
 // 0.37 ms (97 us would be the FP64 pipe's time at its measured 47 TFLOP/s).
+// Orders up to 24 come here from the MFMA and lane families where team_items
+// and lane_team_items say so: M2L of order 8, 500 translations 8.8 -> 5.2 us;
+// order 20, 30,011 124.6 -> 114 us.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -427,10 +430,16 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     squares(kLFwd ? r : rinv);
 
     // ---- forward: scale r^-(n+1) (translations.cpp:45), L2L r^n (:198)
-    auto forward = [&](auto njc, auto oddc, int n, double f, const dbl2(&cr)[NJX], const dbl2(&ci)[NJX]) {
+    // Loads return in order.  Where the operands are held in registers they
+    // are requested before the next degree, so that no swap waits for it;
+    // where they are read again and again it comes first and has the longest
+    // way (order 20 measured 5-8 % slower the other way round).
+    constexpr bool kHeldAll = NJX <= 2;
+    auto forward = [&](auto njc, auto oddc, int n, double f, const dbl2(&cr)[NJX], const dbl2(&ci)[NJX], int next) {
         constexpr int NJ = decltype(njc)::value, ODD = decltype(oddc)::value;
         Operands<NJ> A;
         A.load(tables + (kLFwd ? table_size() : 0), n, lane);
+        if constexpr (kAhead && kHeldAll) load_source(next);
         double xr[2][NJ], xi[2][NJ];
         static_for<0, NJ>([&](auto jc) {
             constexpr int j = decltype(jc)::value;
@@ -464,9 +473,9 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
         dbl2 cr[NJX], ci[NJX];
         if constexpr (!kAhead) load_source(n);
         take(cr, ci);
-        if constexpr (kAhead) load_source(next);
+        if constexpr (kAhead && !kHeldAll) load_source(next);
         const double f = ipow<kBits>(sq, kLFwd ? n : n + 1);
-        by_degree(n, [&](auto njc, auto oddc) { forward(njc, oddc, n, f, cr, ci); });
+        by_degree(n, [&](auto njc, auto oddc) { forward(njc, oddc, n, f, cr, ci, next); });
         n = next;
     }
     // the first target degree is on its way during the z-translation
@@ -485,43 +494,56 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
         if (m >= pout_w) continue;
         const int nk = pin_w - m, nn = pout_w - m;  // input and output degrees
         double2 *top = tri + (column(pc, m) + m) * T + tt;  // degree m
-        double br[2 * NJX], bi[2 * NJX];
-        static_for<0, 2 * NJX>([&](auto cc) {
-            constexpr int c = decltype(cc)::value;
-            br[c] = 0.0;
-            bi[c] = 0.0;
-            if (4 * c < nk) {
-                const bool ok = 4 * c + q < nk;
-                const double2 v = top[(ok ? 4 * c + q : 0) * T];
-                br[c] = ok ? v.x : 0.0;
-                bi[c] = ok ? v.y : 0.0;
-            }
-        });
         const bool flip = OP == SFMM_M2L && (q & 1);  // (-1)^(N+m) of the lane's rows
         auto put = [&](int row, double re, double im) {
             if (row < nn) top[row * T] = double2{flip ? -re : re, flip ? -im : im};
         };
         if constexpr (NJX <= kSmall) {
-            const int i = t & 3;
-            const double *wt = sh + weight_pad(OP) + (OP == SFMM_M2L ? 2 * m + (i + q) : OP == SFMM_M2M ? i - q : q - i);
-            static_for<0, 2 * NJX>([&](auto oc) {
-                constexpr int o = decltype(oc)::value;
-                if (4 * o < nn) {
-                    double dr = 0.0, di = 0.0;
-                    static_for<0, 2 * NJX>([&](auto cc) {
+            const int chunks = (max(nk, nn) + 3) / 4;
+            static_for<1, 2 * NJX + 1>([&](auto ncc) {
+                constexpr int NC = decltype(ncc)::value;
+                if (chunks == NC) {
+                    double br[NC], bi[NC], dr[NC], di[NC], w[2 * NC];
+                    static_for<0, NC>([&](auto cc) {
                         constexpr int c = decltype(cc)::value;
-                        if constexpr (!((OP == SFMM_M2M && c > o) || (OP == SFMM_L2L && c < o))) {
-                            if (4 * c < nk) {
-                                const double w = wt[4 * (OP == SFMM_M2L ? o + c : OP == SFMM_M2M ? o - c : c - o)];
-                                dr = mfma4(w, br[c], dr);
-                                di = mfma4(w, bi[c], di);
-                            }
-                        }
+                        const bool ok = 4 * c + q < nk;
+                        const double2 v = top[(ok ? 4 * c + q : 0) * T];
+                        br[c] = ok ? v.x : 0.0;
+                        bi[c] = ok ? v.y : 0.0;
                     });
-                    put(4 * o + q, dr, di);
+                    const int i = t & 3;
+                    const double *wt =
+                        sh + weight_pad(OP) + (OP == SFMM_M2L ? 2 * m + (i + q) : OP == SFMM_M2M ? i - q : q - i);
+                    static_for<0, OP == SFMM_M2L ? 2 * NC - 1 : NC>(
+                        [&](auto uc) { w[decltype(uc)::value] = wt[4 * decltype(uc)::value]; });
+                    static_for<0, NC>([&](auto cc) {  // 2 NC independent chains
+                        constexpr int c = decltype(cc)::value;
+                        static_for<0, NC>([&](auto oc) {
+                            constexpr int o = decltype(oc)::value;
+                            constexpr int u = OP == SFMM_M2L ? o + c : OP == SFMM_M2M ? o - c : c - o;
+                            if constexpr (u >= 0) {
+                                constexpr bool fresh = OP == SFMM_L2L ? c == o : c == 0;
+                                dr[o] = mfma4(w[u], br[c], fresh ? 0.0 : dr[o]);
+                                di[o] = mfma4(w[u], bi[c], fresh ? 0.0 : di[o]);
+                            }
+                        });
+                    });
+                    static_for<0, NC>([&](auto oc) { put(4 * decltype(oc)::value + q, dr[decltype(oc)::value], di[decltype(oc)::value]); });
                 }
             });
         } else {
+            double br[2 * NJX], bi[2 * NJX];
+            static_for<0, 2 * NJX>([&](auto cc) {
+                constexpr int c = decltype(cc)::value;
+                br[c] = 0.0;
+                bi[c] = 0.0;
+                if (4 * c < nk) {
+                    const bool ok = 4 * c + q < nk;
+                    const double2 v = top[(ok ? 4 * c + q : 0) * T];
+                    br[c] = ok ? v.x : 0.0;
+                    bi[c] = ok ? v.y : 0.0;
+                }
+            });
             const double *wt = sh + weight_pad(OP) + (OP == SFMM_M2L ? 2 * m + (t + q) : OP == SFMM_M2M ? t - q : q - t);
             static_for<0, (NJX + 1) / 2>([&](auto bc) {
                 constexpr int b = decltype(bc)::value;
@@ -553,10 +575,11 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
 
     // ---- backward: scale r^-N (translations.cpp:180), M2M r^(N+1) (:129)
     squares(OP == SFMM_M2M ? r : rinv);
-    auto backward = [&](auto njc, auto oddc, int N, double f, const dbl2(&cr)[NJX], const dbl2(&ci)[NJX]) {
+    auto backward = [&](auto njc, auto oddc, int N, double f, const dbl2(&cr)[NJX], const dbl2(&ci)[NJX], int next) {
         constexpr int NJ = decltype(njc)::value, ODD = decltype(oddc)::value;
         Operands<NJ> A;
         A.load(tables + (kLBwd ? table_size() : 0), N, lane);
+        if constexpr (kAhead && kHeldAll) load_target(next);
         double xr[2][NJ], xi[2][NJ];
         static_for<0, 2 * NJ>([&](auto ic) {
             constexpr int e = decltype(ic)::value & 1, j = decltype(ic)::value >> 1;
@@ -608,9 +631,9 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
         dbl2 cr[NJX], ci[NJX];
         if constexpr (!kAhead) load_target(N);
         take(cr, ci);
-        if constexpr (kAhead) load_target(next);
+        if constexpr (kAhead && !kHeldAll) load_target(next);
         const double f = ipow<kBits>(sq, OP == SFMM_M2M ? N + 1 : N);
-        by_degree(N, [&](auto njc, auto oddc) { backward(njc, oddc, N, f, cr, ci); });
+        by_degree(N, [&](auto njc, auto oddc) { backward(njc, oddc, N, f, cr, ci, next); });
         N = next;
     }
 
@@ -626,6 +649,8 @@ using fn_t = void (*)(const double *, double *, const sfmm_item *, uint32_t, con
 
 // Kernels of one operator, by largest chunk count (team_{m2m,m2l,l2l}.hip).
 struct Kernels {
+    fn_t upto16, upto24;    // four waves
+    fn_t upto16w, upto24w;  // eight waves
     fn_t upto32, upto48;
 };
 template <int OP>

@@ -7,7 +7,8 @@ namespace team {
 template <>
 const Kernels &kernels<SFMM_M2L>()
 {
-    static const Kernels k{&k_team<SFMM_M2L, 4, 4, 8, 2>, &k_team<SFMM_M2L, 6, -1, 8, 2>};
+    static const Kernels k{&k_team<SFMM_M2L, 2, 4, 4, 2>, &k_team<SFMM_M2L, 3, 4, 4, 2>, &k_team<SFMM_M2L, 2, 4, 8, 2>,
+                           &k_team<SFMM_M2L, 3, 4, 8, 2>, &k_team<SFMM_M2L, 4, 4, 8, 2>, &k_team<SFMM_M2L, 6, -1, 8, 2>};
     return k;
 }
 

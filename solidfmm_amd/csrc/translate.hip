@@ -40,6 +40,39 @@ int default_family(uint32_t pb)
     return kGenericKernel;
 }
 
+// The straight-line MFMA kernels give a wave 16 translations from start to
+// end, so a list takes whole rounds of 16,384 (one wave per SIMD): 20 us a
+// round at order 12, 35 at 16, 72 at 20, most of it one wave's chain of
+// degrees and, above order 17, code that outgrows the instruction cache. The
+// team kernel walks the degrees of a group side by side: 9 us for one group
+// and 11 for 4,000 translations at order 12, 11 and 14 at 16, 15 and 21 at 20.
+// It needs more instructions per translation, so the straight-line kernels
+// keep the long lists up to order 20. M2M, straight-line against team (us):
+//   order 12:  8,000 19.1, 15.6;  12,000 20.5, 23.0;  120,000 144, 175
+//   order 16:  12,000 34.3, 32.2;  16,000 35.3, 37.3;  120,000 288, 281
+//   order 18:  12,000 50.6, 45.9;  16,000 51.4, 52.0;  120,000 360, 430
+//   order 20:  24,000 121, 80;  50,000 229, 204;  120,000 452, 472
+//   order 21:  120,000 817, 523;  order 24: 1565, 609
+// (M2L and L2L of order 20 at 120,000: 470, 435 and 450, 428).
+size_t team_items(int op, uint32_t pb)
+{
+    constexpr size_t kAll = ~size_t(0);
+    if (pb <= 14) return 8192;
+    if (pb <= 19) return 12288;
+    if (pb == 20) return op == SFMM_M2M ? 65536 : kAll;
+    return kAll;
+}
+
+// At orders 8 to 11 a team is faster than one lane per translation while the
+// lanes leave most of the chip idle (M2L: order 8, 1,000 items 11.9 -> 8.1
+// us, 4,000 12.4 -> 8.6; order 10 13.9 -> 9.5 and 14.3 -> 10.2; at 8,000 order
+// 10 takes 14.8 and 14.0, L2L 12.4 and 14.0). Below, a lane's chain is as short
+// as a team's (order 7, 4,000: 8.2 and 8.4).
+size_t lane_team_items(uint32_t pb)
+{
+    return pb >= 8 && pb <= kLaneAutoMax ? 4096 : 0;
+}
+
 uint32_t generic_bucket(uint32_t pb)
 {
     if (pb <= uint32_t(mfma::kMfmaMax) || pb > kTeamMax) return kGenericRest;
@@ -150,9 +183,10 @@ hipError_t launch_kernel(int op, const KernelChoice &k, const sfmm_item *items, 
         return hipGetLastError();
     }
     case kMfmaKernels: {
+        const int mode = (!k.acc && k.seg) ? 2 : acc;
+        if (n <= team_items(op, k.pk)) return launch_team(op, k.pk, items, n, src, dst, stream, mode);
         const double *table = mfma::device_table();
         if (!table) return hipErrorOutOfMemory;
-        const int mode = (!k.acc && k.seg) ? 2 : acc;
         return k.rt ? launch_mfma<true>(op, k.pk, items, n, src, dst, table, stream, mode)
                     : launch_mfma<false>(op, k.pk, items, n, src, dst, table, stream, mode);
     }

@@ -13,12 +13,14 @@ namespace sfmm {
 // Kernel families:
 //   lane     one lane per translation, FP64 VALU, orders up to 12
 //            (lane_kernel.hpp);
-//   MFMA     one wave per 16 translations, swaps on the FP64 matrix cores,
-//            orders up to 24 (translate_mfma.hpp);
+//   MFMA     swaps on the FP64 matrix cores, orders up to 24: one wave per
+//            16 translations (translate_mfma.hpp, long lists of orders up to
+//            20) or several (team.hpp);
 //   generic  any orders up to 86: 25 to 48 on the team kernels (team.hpp),
 //            the rest one workgroup per translation (generic.hip).
-// Lane and MFMA kernels are instantiated per square order PB; their RT
-// variants take items of any orders p_in, p_out <= PB.
+// Lane and straight-line MFMA kernels are instantiated per square order PB;
+// their RT variants take items of any orders p_in, p_out <= PB, as the team
+// and generic kernels always do.
 enum Family { kAuto = 0, kLaneKernels = 1, kMfmaKernels = 2, kGenericKernel = 3 };
 
 inline constexpr uint32_t kLaneMax = 12;
@@ -31,6 +33,9 @@ inline constexpr uint32_t kLaneAutoMax = 11;
 namespace mfma {
 inline constexpr int kMfmaMin = 1;
 inline constexpr int kMfmaMax = 24;
+// Orders above this have no kernel in translate_mfma.hpp: the team kernel is
+// faster on every list (team_items).
+inline constexpr int kMfmaKernelMax = 20;
 template <int OP, bool RT>
 hipError_t launch_op(uint32_t P, const sfmm_item *items, size_t n, const double *src, double *dst,
                      const double *table, hipStream_t stream, int acc);
@@ -74,6 +79,13 @@ hipError_t launch_prec_mfma_m2l(uint32_t P, const sfmm_item *items, size_t n, co
 inline constexpr uint32_t kTeamMax = 48;
 hipError_t launch_team(int op, uint32_t pc, const sfmm_item *items, size_t n, const double *src, double *dst,
                        hipStream_t stream, int mode);
+
+// Largest list of orders up to pb that the MFMA family sends to the team
+// kernel instead of the straight-line one (translate.hip has the figures).
+size_t team_items(int op, uint32_t pb);
+// Largest bucket of larger order pb that goes to the MFMA family, and there to
+// the team kernel, although the lane kernels are the default for pb.
+size_t lane_team_items(uint32_t pb);
 
 // Launch bucket of an FP64 item of the generic family, by its larger order:
 // 32 (orders 25 to 32) and kTeamMax (33 to 48) run on team kernels of their

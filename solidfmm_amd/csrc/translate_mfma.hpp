@@ -716,8 +716,8 @@ template <int OP, bool RT>
 hipError_t launch_op(uint32_t P, const sfmm_item *items, size_t n, const double *src, double *dst,
                      const double *table, hipStream_t stream, int acc)
 {
-    static const auto tab = make_table<OP, RT>(std::make_integer_sequence<int, kMfmaMax - kMfmaMin + 1>{});
-    if (P < uint32_t(kMfmaMin) || P > uint32_t(kMfmaMax)) return hipErrorInvalidValue;
+    static const auto tab = make_table<OP, RT>(std::make_integer_sequence<int, kMfmaKernelMax - kMfmaMin + 1>{});
+    if (P < uint32_t(kMfmaMin) || P > uint32_t(kMfmaKernelMax)) return hipErrorInvalidValue;
     const fn_t f = tab.f[P - kMfmaMin];
     const size_t groups = (n + 15) / 16;
     const uint32_t grid =

@@ -1,7 +1,7 @@
 """Team kernels (several waves per group of translations) against the oracle
 -- needs an MI355X.
 
-Orders above 24 run on physical (decaying) expansions.  Error measure: per
+All run on physical (decaying) expansions.  Error measure: per
 item, the 2-norm of the difference over the 2-norm of the oracle's block.
 Bound: 20 times the largest distance of the oracle from the naive O(P^4)
 formulas on the same items (two evaluations of one algorithm, whose errors
@@ -102,3 +102,49 @@ def test_high_orders_repeated_targets(sfmm, orc, P):
     items, src, dst = physical_batch(orc, W.M2L, P, P, 29, 3 * P)
     items["dst"] = (np.arange(29) % 4) * P * (P + 1)
     check(sfmm, orc, W.M2L, items, src, np.zeros(len(dst)), f"repeated P={P}")
+
+
+# Short lists up to order 24, where plans choose between lanes, team and
+# straight-line kernels: orders around 8 chunks' ends (9, 17, 24), 20 | 21 as
+# the last straight-line order, item counts around a group of 16, around 256
+# groups (eight waves a group, then four) and around the dispatch's 4,096
+@pytest.mark.parametrize("op", OPS)
+@pytest.mark.parametrize("P,n", [(8, 1), (8, 4096), (8, 4097), (9, 15), (11, 17), (12, 33), (15, 16), (16, 17),
+                                 (16, 4097), (17, 31), (18, 4113), (20, 16), (21, 49), (24, 18)])
+def test_low_orders_square(sfmm, orc, op, P, n):
+    items, src, dst = physical_batch(orc, op, P, P, n, 7 * P + n + op)
+    dst0 = 1e-3 * np.resize(src, len(dst))
+    check(sfmm, orc, op, items, src, dst0, f"op {op} P={P} n={n}")
+
+
+@pytest.mark.parametrize("op", OPS)
+@pytest.mark.parametrize("family", [0, 2])
+def test_low_orders_mixed(sfmm, orc, op, family):
+    """Order pairs up to 24, zero shifts among them, each target three times
+    in a row (rounds) or eleven times (scratch blocks and runs)."""
+    pairs = [(1, 1), (1, 9), (8, 3), (8, 8), (9, 10), (11, 2), (12, 13), (16, 16), (16, 17), (17, 5), (20, 20),
+             (21, 20), (19, 24), (24, 1)]
+    if op == W.L2L:
+        pairs = [(a, b) for a, b in pairs if a <= b + 1]
+    rng = np.random.default_rng(23 + op)
+    for repeats in (3, 11):
+        items, srcs, so, do = [], [], 0, 0
+        for a, b in pairs:
+            it, s, d = physical_batch(orc, op, a, b, 2 * repeats, 300 + 10 * a + b + op)
+            it = it.copy()
+            it["src"] += np.uint64(so)
+            it["dst"] = np.uint64(do) + np.arange(2 * repeats, dtype=np.uint64) % 2 * np.uint64(b * (b + 1))
+            if op != W.M2L:
+                for c in "xyz":
+                    it[c][a % 5] = 0.0
+            items.append(it)
+            srcs.append(s)
+            so, do = so + len(s), do + len(d)
+        items = rng.permutation(np.concatenate(items))
+        src = np.concatenate(srcs)
+        want = orc.translate(op, items, src, np.zeros(do))
+        naive = orc.translate(op, items, src, np.zeros(do), naive=True)
+        tol = max(20 * block_errors(naive, want, np.zeros(do), items).max(), 1e-13)
+        err = block_errors(run(sfmm, op, items, src, np.zeros(do), family), want, np.zeros(do), items).max()
+        print(f"mixed op {op} family {family} repeats {repeats}: {err:.2e} (tol {tol:.2e})", flush=True)
+        assert err <= tol
