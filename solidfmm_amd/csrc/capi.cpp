@@ -30,6 +30,7 @@
 
 #include "../../include/solidfmm_gpu.h"
 #include "mfma_tables.hpp"
+#include "octet_tables.hpp"
 #include "team_tables.hpp"
 #include "translate.hpp"
 
@@ -223,7 +224,6 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
     keys.reserve(n);
     FlatMap seen;  // target -> occurrences so far
     uint32_t rounds = 0;
-    size_t lanes[kMaxRounds][sfmm::kLaneMax + 1] = {};  // items of the lane kernels per round and order
     // kernel family per (p_in, p_out), filled on first use: lists repeat a
     // handful of order pairs millions of times
     constexpr int kNoKernel = -2, kUnknown = -1;
@@ -256,28 +256,22 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
         uint32_t bucket = pb;
         if (fam == sfmm::kGenericKernel)
             bucket = ctx->precision == SFMM_FP64 ? sfmm::generic_bucket(pb) : sfmm::kGenericRest;
-        if (fam == sfmm::kLaneKernels && pb <= sfmm::kLaneMax) ++lanes[std::min(round, kMaxRounds - 1)][pb];
         keys.push_back({round, fam, bucket, it.p_in, it.p_out, i});
     }
     plan.scratch = rounds > kMaxRounds;
     if (plan.scratch)
         for (Key &k : keys) k.round = 0;
-    // Small buckets of the lane kernels go to the MFMA family's team kernel
-    // where neither the context nor its tuning asks for lanes. Decided here,
-    // before runs are laid out by the family's wave.
-    if (ctx->precision == SFMM_FP64 && ctx->family == SFMM_KERNELS_AUTO) {
-        bool moved[kMaxRounds][sfmm::kLaneMax + 1] = {}, any = false;
-        for (uint32_t pb = 1; pb <= sfmm::kLaneMax; ++pb) {
-            if (plan.scratch)
-                for (uint32_t r = 1; r < kMaxRounds; ++r) lanes[0][pb] += lanes[r][pb];
-            for (uint32_t r = 0; r < (plan.scratch ? 1u : kMaxRounds); ++r) {
-                moved[r][pb] = lanes[r][pb] && !ctx->tune[op][pb] && lanes[r][pb] <= sfmm::lane_team_items(pb);
-                any = any || moved[r][pb];
-            }
-        }
-        if (any)
-            for (Key &k : keys)
-                if (k.family == sfmm::kLaneKernels && moved[k.round][k.pb]) k.family = sfmm::kMfmaKernels;
+    // Long buckets of repeated targets stay on the lane kernels up to
+    // kLaneRunsMax, unless the context or its tuning chooses a family.
+    if (plan.scratch && ctx->precision == SFMM_FP64 && ctx->family == SFMM_KERNELS_AUTO) {
+        size_t count[sfmm::kLaneRunsMax + 1] = {};
+        auto movable = [&](const Key &k) {
+            return k.family == sfmm::kMfmaKernels && k.pb <= sfmm::kLaneRunsMax && !ctx->tune[op][k.pb];
+        };
+        for (const Key &k : keys)
+            if (movable(k)) ++count[k.pb];
+        for (Key &k : keys)
+            if (movable(k) && count[k.pb] > sfmm::team_items(op, k.pb)) k.family = sfmm::kLaneKernels;
     }
     // keys are in list order here: remember each item's position in it
     std::vector<uint32_t> list_pos;
@@ -328,13 +322,14 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
     }
     // FP64 lane and MFMA kernels in scratch mode share one scratch block
     // among the items of a run: consecutive items of a launch, within one
-    // 64-item wave (lane kernels) or 16-item group (MFMA kernels), with the
-    // same target and orders and a nonzero shift (the kernels add a run's
-    // results across lanes).
+    // 64-item wave (lane kernels) or group of 8 (octet kernels) or 16 (team
+    // kernels), with the same target and orders and a nonzero shift (the
+    // kernels add a run's results across lanes).
     const bool runs = plan.scratch && ctx->precision == SFMM_FP64;
     auto zero = [](const sfmm_item &it) { return it.x == 0.0 && it.y == 0.0 && it.z == 0.0; };
     const sfmm_item *prev = nullptr;
     uint64_t run_off = 0;
+    size_t wave = 64;  // items a run of the launch may span
     for (size_t k = 0; k < m; ++k) {
         const Key &key = keys[k];
         if (k == 0 || keys[k - 1].round != key.round || keys[k - 1].family != key.family ||
@@ -342,6 +337,11 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
             plan.launches.push_back(
                 {{key.family, key.family == sfmm::kGenericKernel ? 0u : key.pb, false, ctx->precision, !plan.scratch},
                  ordered.size(), 0, key.round});
+            size_t count = 1;
+            while (k + count < m && keys[k + count].round == key.round && keys[k + count].family == key.family &&
+                   keys[k + count].pb == key.pb)
+                ++count;
+            wave = key.family == sfmm::kLaneKernels ? 64 : count <= sfmm::team_items(op, key.pb) ? 16 : 8;
             plan.launches.back().k.seg =
                 runs && (key.family == sfmm::kLaneKernels || key.family == sfmm::kMfmaKernels);
             prev = nullptr;
@@ -355,7 +355,6 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
         const sfmm_item &src_it = items[key.index];
         sfmm_item it = src_it;
         if (plan.scratch) {
-            const size_t wave = key.family == sfmm::kLaneKernels ? 64 : 16;
             const bool join = L.k.seg && prev && L.count % wave != 0 && prev->dst == src_it.dst &&
                               prev->p_in == src_it.p_in && prev->p_out == src_it.p_out && !zero(*prev) &&
                               !zero(src_it);
@@ -558,7 +557,8 @@ hipError_t ensure_branches(sfmm_context *ctx)
 // allocation happens inside one.
 bool tables_ready()
 {
-    return sfmm::mfma::device_table() && sfmm::mfma::device_factorials() && sfmm::team::device_table();
+    return sfmm::mfma::device_table() && sfmm::mfma::device_factorials() && sfmm::team::device_table() &&
+           sfmm::octet::device_table();
 }
 
 // Device scratch of the allocation-free entry point (sfmm_translate_noalloc):

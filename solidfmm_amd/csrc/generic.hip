@@ -4,7 +4,7 @@
 // index m, the rotated triangle lives in LDS, the folded swap blocks come
 // from the dense device table (mfma_tables.hpp).  This is the complete-
 // coverage path behind the specialised kernels of lane_kernel.hpp,
-// translate_mfma.hpp and team.hpp, which it must agree with: orders above 48,
+// octet.hpp and team.hpp, which it must agree with: orders above 48,
 // and lower ones where a context asks for it.
 //
 // Steps follow translations.cpp:36-471: forward transforms per input degree

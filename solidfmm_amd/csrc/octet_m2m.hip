@@ -1,0 +1,10 @@
+// M2M octet kernels (octet.hpp).
+#include "octet.hpp"
+
+namespace sfmm {
+namespace octet {
+
+template hipError_t launch_op<SFMM_M2M>(uint32_t, const sfmm_item *, size_t, const double *, double *, hipStream_t, int);
+
+}  // namespace octet
+}  // namespace sfmm

@@ -17,6 +17,7 @@
 
 #include "../../include/solidfmm_gpu.h"
 #include "mfma_tables.hpp"
+#include "octet_tables.hpp"
 #include "team_tables.hpp"
 
 namespace sfmm {
@@ -77,6 +78,32 @@ const SwapRecurrence &recurrence()
     }();
     return rec;
 }
+
+// One device copy per device of a table built on the host.
+class DeviceCopies {
+    std::mutex mu;
+    std::vector<double *> per_device;
+
+public:
+    const double *get(std::vector<double> (*build)())
+    {
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+        std::lock_guard<std::mutex> lock(mu);
+        if (per_device.size() <= size_t(dev)) per_device.resize(dev + 1, nullptr);
+        if (!per_device[dev]) {
+            const std::vector<double> h = build();
+            double *d = nullptr;
+            if (hipMalloc(&d, h.size() * sizeof(double)) != hipSuccess) return nullptr;
+            if (hipMemcpy(d, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess) {
+                (void)hipFree(d);
+                return nullptr;
+            }
+            per_device[dev] = d;
+        }
+        return per_device[dev];
+    }
+};
 
 }  // namespace
 
@@ -196,26 +223,46 @@ std::vector<double> build_tables()
 
 const double *device_table()
 {
-    static std::mutex mu;
-    static std::vector<double *> per_device;
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
-    std::lock_guard<std::mutex> lock(mu);
-    if (per_device.size() <= size_t(dev)) per_device.resize(dev + 1, nullptr);
-    if (!per_device[dev]) {
-        const std::vector<double> h = build_tables();
-        double *d = nullptr;
-        if (hipMalloc(&d, h.size() * sizeof(double)) != hipSuccess) return nullptr;
-        if (hipMemcpy(d, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess) {
-            (void)hipFree(d);
-            return nullptr;
-        }
-        per_device[dev] = d;
-    }
-    return per_device[dev];
+    static DeviceCopies copies;
+    return copies.get(build_tables);
 }
 
 }  // namespace team
+
+namespace octet {
+
+namespace {
+
+// Both tables of octet_tables.hpp.
+std::vector<double> build_tables()
+{
+    const SwapRecurrence &rec = recurrence();
+    const int size = table_size(kMaxOrder);
+    std::vector<double> out(2 * size_t(size), 0.0);
+    for (int n = 0; n < kMaxOrder; ++n)
+        for (int part = 0; part < 2; ++part)
+            for (int e = 0; e < 2; ++e) {
+                const int o = (e + n + part) & 1;  // class of the outputs
+                for (int i = 0; 2 * i + o <= n; ++i)
+                    for (int j = 0; 2 * j + e <= n; ++j) {
+                        const int at = entry(n, part, e, i / 4, j / 4, i % 4, j % 4);
+                        const int m = 2 * i + o, l = 2 * j + e;
+                        out[at] = rec.folded(n, part, m, l);
+                        out[size + at] = (l ? 2.0 : 1.0) * (m ? 0.5 : 1.0) * rec.folded(n, part, l, m);
+                    }
+            }
+    return out;
+}
+
+}  // namespace
+
+const double *device_table()
+{
+    static DeviceCopies copies;
+    return copies.get(build_tables);
+}
+
+}  // namespace octet
 }  // namespace sfmm
 
 extern "C" int sfmm_swap_block(int n, int part, double *out)

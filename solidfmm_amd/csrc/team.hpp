@@ -22,15 +22,15 @@
 //
 // Degrees are a run-time loop over a body per chunk count NJ = n/8 + 1 and
 // parity of n, so code does not grow with the order (45 kB at order 32; the
-// straight-line MFMA kernel has 159 kB at order 24, more than the 64 kB
+// straight-line kernel would have 159 kB at order 24, more than the 64 kB
 // instruction cache).  A lone group is bound by its chain of degrees, which
 // the waves walk side by side; a full chip by the FP64 pipe that matrix and
 // vector instructions share.  M2L of order 32: 2,003 translations 577 us on
 // the one-workgroup-per-translation kernel, 37 us here; 30,000 7.7 ms and
 // 0.37 ms (97 us would be the FP64 pipe's time at its measured 47 TFLOP/s).
-// Orders up to 24 come here from the MFMA and lane families where team_items
-// and lane_team_items say so: M2L of order 8, 500 translations 8.8 -> 5.2 us;
-// order 20, 30,011 124.6 -> 114 us.
+// Orders up to 24 come here on lists too short to fill the chip with
+// octet.hpp's groups (team_items): M2L of order 8, 500 translations took 8.8
+// us on lanes and 5.2 here.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -1,7 +1,7 @@
 // Dispatch of the translation kernels: (op, kernel choice) -> launch.
 //
 // The kernels themselves live in lane_kernel.hpp (one lane per
-// translation), translate_mfma.hpp (16 translations per wave on the FP64
+// translation), octet.hpp and team.hpp (8 or 16 translations per group on the FP64
 // matrix cores), team.hpp (up to 16 translations per workgroup, orders 25 to
 // 48), generic.hip (one workgroup per translation, any order) and,
 // for the reduced-precision modes, lane_prec.hpp, mfma_prec.hpp (FP32
@@ -27,7 +27,7 @@ bool family_covers(int family, uint32_t pb)
     if (pb < 1) return false;
     switch (family) {
     case kLaneKernels: return pb <= kLaneMax;
-    case kMfmaKernels: return pb >= uint32_t(mfma::kMfmaMin) && pb <= uint32_t(mfma::kMfmaMax);
+    case kMfmaKernels: return pb <= uint32_t(mfma::kMfmaMax);
     case kGenericKernel: return pb <= uint32_t(mfma::kMaxOrder);
     default: return false;
     }
@@ -40,37 +40,28 @@ int default_family(uint32_t pb)
     return kGenericKernel;
 }
 
-// The straight-line MFMA kernels give a wave 16 translations from start to
-// end, so a list takes whole rounds of 16,384 (one wave per SIMD): 20 us a
-// round at order 12, 35 at 16, 72 at 20, most of it one wave's chain of
-// degrees and, above order 17, code that outgrows the instruction cache. The
-// team kernel walks the degrees of a group side by side: 9 us for one group
-// and 11 for 4,000 translations at order 12, 11 and 14 at 16, 15 and 21 at 20.
-// It needs more instructions per translation, so the straight-line kernels
-// keep the long lists up to order 20. M2M, straight-line against team (us):
-//   order 12:  8,000 19.1, 15.6;  12,000 20.5, 23.0;  120,000 144, 175
-//   order 16:  12,000 34.3, 32.2;  16,000 35.3, 37.3;  120,000 288, 281
-//   order 18:  12,000 50.6, 45.9;  16,000 51.4, 52.0;  120,000 360, 430
-//   order 20:  24,000 121, 80;  50,000 229, 204;  120,000 452, 472
-//   order 21:  120,000 817, 523;  order 24: 1565, 609
-// (M2L and L2L of order 20 at 120,000: 470, 435 and 450, 428).
+// An octet kernel walks a group's degrees in one wave, a team kernel side by
+// side in four or eight: 9 us against 8 for a lone group of order 8, 22
+// against 12 at 16, 42 against 20 at 24. The octet kernel does the same work
+// in fewer cycles, so it takes over once groups fill the chip. M2L, team
+// against octet (us):
+//   order  8: 4,096 8.5, 9.3;   8,192 10.8, 9.8;   120,000 99, 46
+//   order 12: 4,096 11.4, 13.5; 8,192 15.7, 14.6;  120,000 178, 101
+//   order 16: 8,192 22.6, 25.7; 12,288 33.2, 26.4; 120,000 288, 204
+//   order 18: 8,192 27.9, 27.3; 12,288 41.8, 41.8; 120,000 378, 288
+//   order 20: 12,288 45.7, 53.0; 24,000 76.5, 76.1; 120,000 425, 365
+//   order 22: 30,011 122, 123;  60,000 266, 242
+//   order 24: 60,000 299, 344;  120,000 584, 626
+// M2M and L2L keep one operand table instead of two and cross over earlier
+// from order 19 (M2M of order 20: 8,192 29.9, 29.0; 12,288 44.8, 45.5;
+// 16,384 51.8, 46.5; order 24: 16,384 67.8, 68.1; 24,000 96.6, 94.4).
 size_t team_items(int op, uint32_t pb)
 {
-    constexpr size_t kAll = ~size_t(0);
-    if (pb <= 14) return 8192;
-    if (pb <= 19) return 12288;
-    if (pb == 20) return op == SFMM_M2M ? 65536 : kAll;
-    return kAll;
-}
-
-// At orders 8 to 11 a team is faster than one lane per translation while the
-// lanes leave most of the chip idle (M2L: order 8, 1,000 items 11.9 -> 8.1
-// us, 4,000 12.4 -> 8.6; order 10 13.9 -> 9.5 and 14.3 -> 10.2; at 8,000 order
-// 10 takes 14.8 and 14.0, L2L 12.4 and 14.0). Below, a lane's chain is as short
-// as a team's (order 7, 4,000: 8.2 and 8.4).
-size_t lane_team_items(uint32_t pb)
-{
-    return pb >= 8 && pb <= kLaneAutoMax ? 4096 : 0;
+    if (pb <= 13) return 6144;
+    if (pb <= 18) return 8192;
+    if (op != SFMM_M2L) return 12288;
+    if (int(pb) > octet::max_order(op)) return ~size_t(0);
+    return pb <= 20 ? 24576 : 32768;
 }
 
 uint32_t generic_bucket(uint32_t pb)
@@ -87,7 +78,7 @@ bool have_kernel(int op, uint32_t p_in, uint32_t p_out, int family)
     return family_covers(family, pb);
 }
 
-uint32_t persistent_grid(const void *kernel, int block, size_t work)
+uint32_t persistent_grid(const void *kernel, int block, size_t work, size_t lds)
 {
     struct Key {
         const void *k;
@@ -106,7 +97,7 @@ uint32_t persistent_grid(const void *kernel, int block, size_t work)
             int per_cu = 0, cus = 0;
             // a failed query falls back to one workgroup per CU; its error
             // is cleared so the launch that follows does not report it
-            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, block, 0) != hipSuccess || per_cu < 1) {
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, block, lds) != hipSuccess || per_cu < 1) {
                 (void)hipGetLastError();
                 per_cu = 1;
             }
@@ -135,21 +126,6 @@ uint32_t lane_items_per_wave(const void *kernel, size_t n)
     const size_t ipw = (n + rounds * slots - 1) / (rounds * slots);
     return uint32_t(ipw < 1 ? 1 : ipw > 64 ? 64 : ipw);
 }
-
-namespace {
-
-template <bool RT>
-hipError_t launch_mfma(int op, uint32_t pk, const sfmm_item *items, size_t n, const double *src, double *dst,
-                       const double *table, hipStream_t stream, int acc)
-{
-    switch (op) {
-    case SFMM_M2M: return mfma::launch_op<SFMM_M2M, RT>(pk, items, n, src, dst, table, stream, acc);
-    case SFMM_M2L: return mfma::launch_op<SFMM_M2L, RT>(pk, items, n, src, dst, table, stream, acc);
-    default: return mfma::launch_op<SFMM_L2L, RT>(pk, items, n, src, dst, table, stream, acc);
-    }
-}
-
-}  // namespace
 
 hipError_t launch_kernel(int op, const KernelChoice &k, const sfmm_item *items, size_t n, const double *src,
                          double *dst, hipStream_t stream)
@@ -185,10 +161,11 @@ hipError_t launch_kernel(int op, const KernelChoice &k, const sfmm_item *items, 
     case kMfmaKernels: {
         const int mode = (!k.acc && k.seg) ? 2 : acc;
         if (n <= team_items(op, k.pk)) return launch_team(op, k.pk, items, n, src, dst, stream, mode);
-        const double *table = mfma::device_table();
-        if (!table) return hipErrorOutOfMemory;
-        return k.rt ? launch_mfma<true>(op, k.pk, items, n, src, dst, table, stream, mode)
-                    : launch_mfma<false>(op, k.pk, items, n, src, dst, table, stream, mode);
+        switch (op) {
+        case SFMM_M2M: return octet::launch_op<SFMM_M2M>(k.pk, items, n, src, dst, stream, mode);
+        case SFMM_M2L: return octet::launch_op<SFMM_M2L>(k.pk, items, n, src, dst, stream, mode);
+        default: return octet::launch_op<SFMM_L2L>(k.pk, items, n, src, dst, stream, mode);
+        }
     }
     default:
         // Orders above the MFMA kernels' 24 run on the team kernels as far

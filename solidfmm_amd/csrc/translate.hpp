@@ -14,31 +14,30 @@ namespace sfmm {
 //   lane     one lane per translation, FP64 VALU, orders up to 12
 //            (lane_kernel.hpp);
 //   MFMA     swaps on the FP64 matrix cores, orders up to 24: one wave per
-//            16 translations (translate_mfma.hpp, long lists of orders up to
-//            20) or several (team.hpp);
+//            eight translations (octet.hpp, long lists) or several waves per
+//            sixteen (team.hpp);
 //   generic  any orders up to 86: 25 to 48 on the team kernels (team.hpp),
 //            the rest one workgroup per translation (generic.hip).
-// Lane and straight-line MFMA kernels are instantiated per square order PB;
-// their RT variants take items of any orders p_in, p_out <= PB, as the team
-// and generic kernels always do.
+// Lane and octet kernels are instantiated per order bound PB.  Lane kernels
+// take items of orders (PB, PB), their RT variants any p_in, p_out <= PB, as
+// all other kernels do.
 enum Family { kAuto = 0, kLaneKernels = 1, kMfmaKernels = 2, kGenericKernel = 3 };
 
 inline constexpr uint32_t kLaneMax = 12;
-// lane kernels by default up to this order: at 11 they beat MFMA on 1e5
-// independent translations (M2L 1.18e9 against 1.04e9/s, M2M 1.37e9
-// against 1.15e9, L2L 1.36e9 against 1.05e9); at 12 MFMA wins (M2L 8.9e8
-// against 6.1e8)
-inline constexpr uint32_t kLaneAutoMax = 11;
+// lane kernels by default up to this order: at 7 they are level with the
+// octet kernels on long lists (M2L of 200,000: 63.1 us on lanes, 62.9), at 8
+// and from 10 up behind (8: 137 against 71; 9: 105, 104; 10: 156, 129; 11:
+// 211, 149), and on short lists of order 8 behind the team kernels (1,000:
+// 11.9 against 8.1; order 7, 4,000: 8.2, 8.4)
+inline constexpr uint32_t kLaneAutoMax = 7;
+// ... and up to this one on long lists of repeated targets: a lane wave adds
+// runs of up to 64 items before it stores, an octet group runs of up to 8
+// (interaction lists of a grid of 14^3 cells, M2L with its reduction: order 8
+// 111 us on lanes, 150 on octets; 10: 213, 230; 11: 265, 267; 12: 368, 299).
+inline constexpr uint32_t kLaneRunsMax = 11;
 
 namespace mfma {
-inline constexpr int kMfmaMin = 1;
 inline constexpr int kMfmaMax = 24;
-// Orders above this have no kernel in translate_mfma.hpp: the team kernel is
-// faster on every list (team_items).
-inline constexpr int kMfmaKernelMax = 20;
-template <int OP, bool RT>
-hipError_t launch_op(uint32_t P, const sfmm_item *items, size_t n, const double *src, double *dst,
-                     const double *table, hipStream_t stream, int acc);
 }  // namespace mfma
 
 // Highest order with a kernel.
@@ -56,7 +55,8 @@ bool have_kernel(int op, uint32_t p_in, uint32_t p_out, int family = kAuto);
 
 // Workgroups for a persistent kernel: as many as can be resident on the
 // current device at once, but no more than `work` (one per unit of work).
-uint32_t persistent_grid(const void *kernel, int block, size_t work);
+// `lds` is the dynamic LDS of a workgroup.
+uint32_t persistent_grid(const void *kernel, int block, size_t work, size_t lds = 0);
 
 // Reduced-precision kernels (arithmetic policies of prec.hpp): a lane
 // kernel for square M2L up to kPrecLaneMax and a generic kernel for every
@@ -80,12 +80,19 @@ inline constexpr uint32_t kTeamMax = 48;
 hipError_t launch_team(int op, uint32_t pc, const sfmm_item *items, size_t n, const double *src, double *dst,
                        hipStream_t stream, int mode);
 
+// Octet kernels (octet.hpp): items of any orders up to pb <= max_order(OP);
+// mode as there.
+namespace octet {
+// M2L lists above it all go to the team kernels (team_items)
+constexpr int max_order(int op) { return op == SFMM_M2L ? 22 : 24; }
+template <int OP>
+hipError_t launch_op(uint32_t pb, const sfmm_item *items, size_t n, const double *src, double *dst,
+                     hipStream_t stream, int mode);
+}  // namespace octet
+
 // Largest list of orders up to pb that the MFMA family sends to the team
-// kernel instead of the straight-line one (translate.hip has the figures).
+// kernel instead of the octet kernel (translate.hip has the figures).
 size_t team_items(int op, uint32_t pb);
-// Largest bucket of larger order pb that goes to the MFMA family, and there to
-// the team kernel, although the lane kernels are the default for pb.
-size_t lane_team_items(uint32_t pb);
 
 // Launch bucket of an FP64 item of the generic family, by its larger order:
 // 32 (orders 25 to 32) and kTeamMax (33 to 48) run on team kernels of their
