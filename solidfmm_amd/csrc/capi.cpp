@@ -271,7 +271,7 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
         for (const Key &k : keys)
             if (movable(k)) ++count[k.pb];
         for (Key &k : keys)
-            if (movable(k) && count[k.pb] > sfmm::team_items(op, k.pb)) k.family = sfmm::kLaneKernels;
+            if (movable(k) && count[k.pb] > sfmm::kLaneRunsItems) k.family = sfmm::kLaneKernels;
     }
     // keys are in list order here: remember each item's position in it
     std::vector<uint32_t> list_pos;

@@ -233,9 +233,19 @@ __device__ __forceinline__ void zero_shift_add(const double *__restrict__ S, dou
 // results by a fixed tree of shuffles and the run's first lane stores the
 // sum, so a run of k items writes one block instead of k.
 struct Segments {
-    uint32_t same = 0;  // bit j: lane + 2^j belongs to this lane's run
-    bool head = true;   // this lane stores its run's sum
+    uint32_t same = 0;   // bit j: lane + 2^j belongs to this lane's run
+    bool head = true;    // this lane stores its run's sum
+    uint64_t heads = 0;  // first lanes of the wave's runs where it has few (run_sums)
 };
+// Waves of at most this many runs add them through LDS.  The tree of
+// shuffles costs the same for any runs, the LDS sums some 15 instructions a
+// run and degree: equal at about 16.
+inline constexpr int kFewRuns = 8;
+// doubles per lane of the LDS copy of one degree (odd: no bank conflicts),
+// and beyond the last lane
+template <int P>
+inline constexpr int kSumStride = 2 * P + 1;
+inline constexpr int kSumPad = 32;
 
 __device__ __forceinline__ double shfl_down(double v, int d)
 {
@@ -278,6 +288,59 @@ __device__ __forceinline__ void segment_sum(const Segments &g, double (&re)[N + 
     });
 }
 
+// Sums of degree N over the runs of a full wave, through LDS: every lane
+// writes its 2 N + 2 reals, then 16 lanes (32 above degree 7) add one real
+// each over every fourth (second) lane of a run, and the run's block is
+// stored as whole lines.  `on`: this lane's run has degree N.  In order-8
+// interaction lists, with runs of up to 64 items, 864 shuffles a wave become
+// 232 LDS accesses, and M2L with its reduction goes from 100.5 to 71.3 us
+// (14^3 cells; order 10: 213 -> 145, order 12: 368 -> 232).
+template <int N, int ST>
+__device__ __forceinline__ void run_sums(const Segments &g, double *buf, double *D, const double (&re)[N + 1],
+                                         const double (&im)[N + 1], bool on)
+{
+    constexpr int CW = N <= 7 ? 16 : 32, G = 64 / CW;
+    const int lane = static_cast<int>(threadIdx.x & 63), c = lane % CW, h = lane / CW;
+    auto fence = [] {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+    fence();
+    double *own = buf + lane * ST;
+    static_for<0, N + 1>([&](auto mc) {
+        constexpr int m = decltype(mc)::value;
+        own[m] = re[m];
+        own[N + 1 + m] = im[m];
+    });
+    fence();
+    const uint64_t target = reinterpret_cast<uint64_t>(D);
+    const uint64_t stored = __ballot(on);
+    for (uint64_t left = g.heads; left;) {  // wave-uniform
+        const int a = __builtin_ctzll(left);
+        left &= left - 1;
+        const int b = left ? __builtin_ctzll(left) : 64;
+        if (!((stored >> a) & 1u)) continue;
+        const double *from = buf + (a + h) * ST + c;
+        double sum = 0.0;
+        int k = 0;
+        for (; k + 4 * G <= b - a; k += 4 * G) {
+            double v[4];
+            static_for<0, 4>([&](auto uc) { v[decltype(uc)::value] = from[(k + G * decltype(uc)::value) * ST]; });
+            sum += (v[0] + v[1]) + (v[2] + v[3]);
+        }
+        for (; k < b - a; k += G) {
+            const bool in = k + h < b - a;
+            const double v = *(in ? from + k * ST : buf + c);
+            sum += in ? v : 0.0;
+        }
+        for (int d = CW; d < 64; d *= 2) sum += __shfl_xor(sum, d, 64);
+        const uint32_t lo = __builtin_amdgcn_readlane(uint32_t(target), a);
+        const uint32_t hi = __builtin_amdgcn_readlane(uint32_t(target >> 32), a);
+        double *to = reinterpret_cast<double *>(uint64_t(hi) << 32 | lo);
+        if (h == 0 && c < 2 * N + 2) to[N * (N + 1) + c] = sum;
+    }
+}
+
 // One lane, one translation (see the head of this file for RT).  acc = 1:
 // target += T(source); acc = 0: target = T(source) over the degrees the
 // translation defines (scratch blocks of a segmented reduction); acc = 2:
@@ -302,6 +365,8 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kLaneWa
     static_assert(!RT || PI == PO, "runtime orders use a square bound");
     constexpr int PM = PI > PO ? PI : PO;
     constexpr int PE = PI < PO ? PI : PO;
+    // a degree of the wave's results, for run_sums
+    __shared__ double sums[RT ? 64 * kSumStride<PI> + kSumPad : 1];
     const uint32_t lane_id = threadIdx.x;
     const uint32_t t = lane_id < ipw ? blockIdx.x * ipw + lane_id : n_items;
     // runs (acc == 2) exist in the per-item-order kernels only; the plan
@@ -338,6 +403,10 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kLaneWa
         y = -y;
         z = -z;
     }
+    if constexpr (RT) {
+        const uint64_t heads = __ballot(seg.head);
+        if (acc == 2 && __ballot(true) == ~uint64_t(0) && __popcll(heads) <= kFewRuns) seg.heads = heads;
+    }
     // Wave-uniform bounds of the degrees worth computing.
     const uint32_t pin_w = RT ? wave_max7(pin) : uint32_t(PI);
     const uint32_t pout_w = RT ? wave_max7(OP == SFMM_L2L ? pend : pout) : uint32_t(PO);
@@ -350,6 +419,10 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kLaneWa
         constexpr int N = decltype(Nc)::value;
         if constexpr (RT) {
             if (acc == 2) {
+                if (seg.heads) {
+                    run_sums<N, kSumStride<PI>>(seg, sums, D, re, im, on);
+                    return;
+                }
                 segment_sum<N>(seg, re, im);
                 on = on && seg.head;
             }

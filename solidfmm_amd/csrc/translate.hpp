@@ -30,11 +30,14 @@ inline constexpr uint32_t kLaneMax = 12;
 // 211, 149), and on short lists of order 8 behind the team kernels (1,000:
 // 11.9 against 8.1; order 7, 4,000: 8.2, 8.4)
 inline constexpr uint32_t kLaneAutoMax = 7;
-// ... and up to this one on long lists of repeated targets: a lane wave adds
-// runs of up to 64 items before it stores, an octet group runs of up to 8
-// (interaction lists of a grid of 14^3 cells, M2L with its reduction: order 8
-// 111 us on lanes, 150 on octets; 10: 213, 230; 11: 265, 267; 12: 368, 299).
-inline constexpr uint32_t kLaneRunsMax = 11;
+// ... and up to this one on lists of repeated targets with more than
+// kLaneRunsItems items: a lane wave adds runs of up to 64 items before it
+// stores, an octet group runs of up to 8, but 64 items a wave need long lists
+// to fill the chip.  Interaction lists of grids, M2L with its reduction, lanes
+// against octets (us): order 8, 29,078 items 26.1, 23.2; 53,352 29.2, 32.7;
+// 374,976 79, 150; order 12 49.9, 43.4; 56.0, 61.2; 232, 302.
+inline constexpr uint32_t kLaneRunsMax = kLaneMax;
+inline constexpr size_t kLaneRunsItems = 40000;
 
 namespace mfma {
 inline constexpr int kMfmaMax = 24;
