@@ -228,6 +228,8 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
     // handful of order pairs millions of times
     constexpr int kNoKernel = -2, kUnknown = -1;
     std::vector<int8_t> fam_of(size_t(ctx->P + 1) * (ctx->P + 1), int8_t(kUnknown));
+    const bool small_m2l = op == SFMM_M2L && n <= sfmm::kLaneSmallM2L && ctx->precision == SFMM_FP64 &&
+                           ctx->family == SFMM_KERNELS_AUTO;
     for (size_t i = 0; i < n; ++i) {
         const sfmm_item &it = items[i];
         if (it.p_in > ctx->P || it.p_out > ctx->P)
@@ -245,8 +247,8 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
             return fail(ctx, SFMM_ERR_UNSUPPORTED,
                         std::string("solidfmm: no kernel for ") + op_name(op) + " with p_in=" +
                             std::to_string(it.p_in) + ", p_out=" + std::to_string(it.p_out));
-        const int fam = fc;
         const uint32_t pb = std::max(it.p_in, it.p_out);
+        const int fam = small_m2l && pb >= 9 && pb <= 11 && !ctx->tune[op][pb] ? sfmm::kLaneKernels : fc;
         bool fresh;
         const uint32_t round = seen.get(it.dst, 0, fresh)++;
         rounds = std::max(rounds, round + 1);

@@ -96,3 +96,21 @@ def test_octet_runs(sfmm, orc, op, P):
         for c in "xyz":
             items[c][3:400:11] = 0.0
     check(sfmm, orc, op, items, src, np.zeros(nd), f"runs op {op} P={P} n={len(items)}")
+
+
+@pytest.mark.parametrize("P", [8, 9, 11, 12])
+@pytest.mark.parametrize("n", [512, 513])
+def test_small_m2l_default(sfmm, orc, P, n):
+    """Both sides of the item count up to which M2L of orders 9 to 11 stays on
+    lanes."""
+    items, src, dst = physical_batch(orc, W.M2L, P, P, n, P + n)
+    ctx = sfmm.Context(P)
+    plan = sfmm.Plan(ctx, W.M2L, items)
+    assert plan.launch_info()[0][0] == (1 if n == 512 and 9 <= P <= 11 else MFMA)
+    d = torch.zeros(len(dst), dtype=torch.float64, device="cuda")
+    plan.execute(torch.from_numpy(src).to("cuda"), d)
+    torch.cuda.synchronize()
+    want = orc.translate(W.M2L, items, src, np.zeros(len(dst)))
+    naive = orc.translate(W.M2L, items, src, np.zeros(len(dst)), naive=True)
+    tol = max(20 * block_errors(naive, want, np.zeros(len(dst)), items).max(), 1e-13)
+    assert block_errors(d.cpu().numpy(), want, np.zeros(len(dst)), items).max() <= tol
