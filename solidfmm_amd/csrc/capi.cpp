@@ -210,7 +210,9 @@ private:
 // are applied in list order by rounds (the k-th item of a target runs in
 // launch round k); otherwise every item writes its own scratch block and a
 // segmented reduction adds a target's blocks in list order (reduce.hip).
-int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm_plan &plan)
+// `compact`: repeated targets run on the kernels of the longest runs the
+// family has, for the fewest scratch blocks.
+int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm_plan &plan, bool compact)
 {
     if (op < SFMM_M2M || op > SFMM_L2L) return fail(ctx, SFMM_ERR_LOGIC, "solidfmm: unknown operator");
     if (n && !items) return fail(ctx, SFMM_ERR_LOGIC, "solidfmm: null item list");
@@ -343,7 +345,9 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
             while (k + count < m && keys[k + count].round == key.round && keys[k + count].family == key.family &&
                    keys[k + count].pb == key.pb)
                 ++count;
-            wave = key.family == sfmm::kLaneKernels ? 64 : count <= sfmm::team_items(op, key.pb) ? 16 : 8;
+            const bool team = compact || count <= sfmm::team_items(op, key.pb);
+            wave = key.family == sfmm::kLaneKernels ? 64 : team ? 16 : 8;
+            plan.launches.back().k.compact = compact && plan.scratch;
             plan.launches.back().k.seg =
                 runs && (key.family == sfmm::kLaneKernels || key.family == sfmm::kMfmaKernels);
             prev = nullptr;
@@ -669,13 +673,13 @@ namespace {
 
 // Validation and grouping into a new plan with no device memory yet (its
 // device image stays on the host).
-int prepare_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm_plan **out)
+int prepare_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm_plan **out, bool compact = false)
 {
     sfmm_plan *plan = new (std::nothrow) sfmm_plan;
     if (!plan) return fail(ctx, SFMM_ERR_ALLOC, "solidfmm: out of host memory");
     int rc;
     try {
-        rc = build_plan(ctx, op, items, n, *plan);
+        rc = build_plan(ctx, op, items, n, *plan, compact);
     } catch (const std::bad_alloc &) {
         rc = fail(ctx, SFMM_ERR_ALLOC, "solidfmm: out of host memory");
     }
@@ -902,6 +906,11 @@ int sfmm_translate_noalloc(sfmm_context *ctx, int op, const sfmm_item *host_item
     int rc = sfmm_plan_prepare(ctx, op, host_items, n, &plan);  // host memory only
     if (rc != SFMM_OK) return rc;
     std::lock_guard<std::mutex> lock(ctx->mu);
+    if (plan->dev_bytes > kNoAllocBytes && plan->scratch) {
+        delete plan;
+        rc = prepare_plan(ctx, op, host_items, n, &plan, true);
+        if (rc != SFMM_OK) return rc;
+    }
     if (plan->dev_bytes > kNoAllocBytes) {
         rc = fail(ctx, SFMM_ERR_LOGIC,
                   "solidfmm: the list needs " + std::to_string(plan->dev_bytes) +

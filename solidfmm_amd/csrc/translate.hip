@@ -160,7 +160,7 @@ hipError_t launch_kernel(int op, const KernelChoice &k, const sfmm_item *items, 
     }
     case kMfmaKernels: {
         const int mode = (!k.acc && k.seg) ? 2 : acc;
-        if (n <= team_items(op, k.pk)) return launch_team(op, k.pk, items, n, src, dst, stream, mode);
+        if (k.compact || n <= team_items(op, k.pk)) return launch_team(op, k.pk, items, n, src, dst, stream, mode);
         switch (op) {
         case SFMM_M2M: return octet::launch_op<SFMM_M2M>(k.pk, items, n, src, dst, stream, mode);
         case SFMM_M2L: return octet::launch_op<SFMM_M2L>(k.pk, items, n, src, dst, stream, mode);

@@ -124,8 +124,11 @@ struct KernelChoice {
     int precision = SFMM_FP64;
     bool acc = true;
     // scratch mode with runs of one target's items sharing a block (FP64
-    // lane kernels only; the plan lays the runs out)
+    // lane, team and octet kernels; the plan lays the runs out)
     bool seg = false;
+    // team kernels for any number of items (their runs are twice as long as
+    // the octet kernels')
+    bool compact = false;
 };
 
 // Segmented reduction: target block t += sum of its items' scratch blocks,

@@ -114,3 +114,31 @@ def test_small_m2l_default(sfmm, orc, P, n):
     naive = orc.translate(W.M2L, items, src, np.zeros(len(dst)), naive=True)
     tol = max(20 * block_errors(naive, want, np.zeros(len(dst)), items).max(), 1e-13)
     assert block_errors(d.cpu().numpy(), want, np.zeros(len(dst)), items).max() <= tol
+
+
+def test_noalloc_long_runs(sfmm, orc):
+    """Repeated targets whose blocks fit the fixed scratch array with runs of
+    16 items, not of 8: M2L of order 16, 240,000 items (all but 200 of them
+    of orders (1, 16)) in runs of 16."""
+    import ctypes
+    n, P = 240000, 16
+    parts = [physical_batch(orc, W.M2L, P, P, 200, 1), physical_batch(orc, W.M2L, 1, P, n - 200, 2)]
+    items, src, nd = join(parts)
+    rep = 16 * 20
+    items["dst"] = (np.arange(n) // rep).astype(np.uint64) * np.uint64(P * (P + 1))
+    order = np.lexsort((np.arange(n), items["p_in"]))
+    items = items[order]
+    nd = (n // rep + 1) * P * (P + 1)
+    ctx = sfmm.Context(P)
+    s, d = torch.from_numpy(src).to("cuda"), torch.zeros(nd, dtype=torch.float64, device="cuda")
+    items = np.ascontiguousarray(items, dtype=W.ITEM_DTYPE)
+    rc = sfmm.load().sfmm_translate_noalloc(ctx.handle, W.M2L, items.ctypes.data, n, s.data_ptr(), s.numel(),
+                                            d.data_ptr(), d.numel(),
+                                            ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0
+    e = torch.zeros_like(d)
+    sfmm.Plan(ctx, W.M2L, items).execute(s, e)
+    torch.cuda.synchronize()
+    # sums of 320 results of one operator in two groupings: 1e-12 of the block
+    a, b = d.cpu().numpy().reshape(-1, P * (P + 1)), e.cpu().numpy().reshape(-1, P * (P + 1))
+    assert (np.linalg.norm(a - b, axis=1) <= 1e-12 * np.linalg.norm(b, axis=1) + 0.0).all()
