@@ -474,7 +474,9 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
         if constexpr (!kAhead) load_source(n);
         take(cr, ci);
         if constexpr (kAhead && !kHeldAll) load_source(next);
-        const double f = ipow<kBits>(sq, kLFwd ? n : n + 1);
+        // a degree that a translation does not have is zero, whatever the
+        // power of r that only longer translations of the group reach
+        const double f = n < pin ? ipow<kBits>(sq, kLFwd ? n : n + 1) : 0.0;
         by_degree(n, [&](auto njc, auto oddc) { forward(njc, oddc, n, f, cr, ci, next); });
         n = next;
     }
@@ -497,6 +499,38 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
         const bool flip = OP == SFMM_M2L && (q & 1);  // (-1)^(N+m) of the lane's rows
         auto put = [&](int row, double re, double im) {
             if (row < nn) top[row * T] = double2{flip ? -re : re, flip ? -im : im};
+        };
+        // M2M and L2L couple a degree with the degrees on one side of it.
+        // The matrix product has zero weights for the others, which an
+        // infinity or a NaN would turn into NaN: such columns are summed
+        // degree by degree.  Looking for them costs 0.5 us of the 8 to 14 of
+        // a short launch (FMM of 100,000 points 872 -> 880 us).
+        auto one_sided = [&] {
+            for (int k4 = 0; 4 * k4 < nn; ++k4) {
+                const int N0 = OP == SFMM_M2M ? 4 * ((nn - 1) / 4 - k4) : 4 * k4;  // read before it is replaced
+                const int N = N0 + q, end = OP == SFMM_M2M ? min(nk, N0 + 4) : nk;
+                double re = 0.0, im = 0.0;
+                for (int K = OP == SFMM_M2M ? 0 : N0; K < end; ++K) {
+                    const double2 v = top[K * T];
+                    const double w = sh[weight_pad(OP) + (OP == SFMM_M2M ? N - K : K - N)];
+                    const bool on = OP == SFMM_M2M ? K <= N : K >= N;
+                    re = on ? __builtin_fma(w, v.x, re) : re;
+                    im = on ? __builtin_fma(w, v.y, im) : im;
+                }
+                __builtin_amdgcn_wave_barrier();
+                put(N, re, im);
+            }
+        };
+        // true where any value of the column is infinite or NaN; integer
+        // instructions between the products, which have the FP64 pipe
+        auto unbounded = [&](const auto &re, const auto &im) {
+            uint32_t top_bits = 0;
+            static_for<0, int(sizeof(re) / sizeof(double))>([&](auto cc) {
+                const double v[2] = {re[decltype(cc)::value], im[decltype(cc)::value]};
+                for (int i = 0; i < 2; ++i)
+                    top_bits = max(top_bits, uint32_t(__builtin_bit_cast(uint64_t, v[i]) >> 32) & 0x7fffffffu);
+            });
+            return OP != SFMM_M2L && __ballot(top_bits >= 0x7ff00000u) != 0;
         };
         if constexpr (NJX <= kSmall) {
             const int chunks = (max(nk, nn) + 3) / 4;
@@ -528,6 +562,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
                             }
                         });
                     });
+                    if (unbounded(br, bi)) return one_sided();
                     static_for<0, NC>([&](auto oc) { put(4 * decltype(oc)::value + q, dr[decltype(oc)::value], di[decltype(oc)::value]); });
                 }
             });
@@ -544,6 +579,10 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
                     bi[c] = ok ? v.y : 0.0;
                 }
             });
+            if (unbounded(br, bi)) {
+                one_sided();
+                continue;
+            }
             const double *wt = sh + weight_pad(OP) + (OP == SFMM_M2L ? 2 * m + (t + q) : OP == SFMM_M2M ? t - q : q - t);
             static_for<0, (NJX + 1) / 2>([&](auto bc) {
                 constexpr int b = decltype(bc)::value;
