@@ -103,6 +103,12 @@ int family_for(const sfmm_context *ctx, int op, uint32_t pb)
     return t ? t : sfmm::default_family(pb);
 }
 
+// Whether orders 25 to 48 of the generic family run on the team kernels.
+bool generic_on_teams(const sfmm_context *ctx)
+{
+    return ctx->precision == SFMM_FP64 && ctx->family != SFMM_KERNELS_GENERIC;
+}
+
 // Kernel for one item on a context: family and whether it has one.  FP64
 // contexts: the family of its bucket max(p_in, p_out).  Reduced-precision
 // contexts, square M2L: the precision lane kernel up to kPrecLaneAutoMax
@@ -230,6 +236,7 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
     // handful of order pairs millions of times
     constexpr int kNoKernel = -2, kUnknown = -1;
     std::vector<int8_t> fam_of(size_t(ctx->P + 1) * (ctx->P + 1), int8_t(kUnknown));
+    const bool team_generic = generic_on_teams(ctx);
     const bool small_m2l = op == SFMM_M2L && n <= sfmm::kLaneSmallM2L && ctx->precision == SFMM_FP64 &&
                            ctx->family == SFMM_KERNELS_AUTO;
     for (size_t i = 0; i < n; ++i) {
@@ -259,7 +266,7 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
         // the generic kernels take many orders in one launch
         uint32_t bucket = pb;
         if (fam == sfmm::kGenericKernel)
-            bucket = ctx->precision == SFMM_FP64 ? sfmm::generic_bucket(pb) : sfmm::kGenericRest;
+            bucket = team_generic ? sfmm::generic_bucket(pb) : sfmm::kGenericRest;
         keys.push_back({round, fam, bucket, it.p_in, it.p_out, i});
     }
     plan.scratch = rounds > kMaxRounds;
@@ -345,9 +352,11 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
             while (k + count < m && keys[k + count].round == key.round && keys[k + count].family == key.family &&
                    keys[k + count].pb == key.pb)
                 ++count;
-            const bool team = compact || count <= sfmm::team_items(op, key.pb);
+            const bool team = key.family == sfmm::kGenericKernel
+                                  ? key.pb != sfmm::kGenericRest
+                                  : (compact && plan.scratch) || count <= sfmm::team_items(op, key.pb);
             wave = key.family == sfmm::kLaneKernels ? 64 : team ? 16 : 8;
-            plan.launches.back().k.compact = compact && plan.scratch;
+            plan.launches.back().k.team = team;
             plan.launches.back().k.seg =
                 runs && (key.family == sfmm::kLaneKernels || key.family == sfmm::kMfmaKernels);
             prev = nullptr;
@@ -1013,7 +1022,11 @@ int sfmm_launch(sfmm_context *ctx, int op, uint32_t p_in, uint32_t p_out, const 
     hipError_t e = hipSetDevice(ctx->device);
     if (e != hipSuccess) return hip_fail(ctx, e, "hipSetDevice");
     const uint32_t pb = std::max(p_in, p_out);
-    const sfmm::KernelChoice k{fam, pb, p_in != p_out, ctx->precision};
+    sfmm::KernelChoice k{fam, pb, p_in != p_out, ctx->precision};
+    if (ctx->precision == SFMM_FP64)
+        k.team = fam == sfmm::kGenericKernel
+                     ? generic_on_teams(ctx) && sfmm::generic_bucket(pb) != sfmm::kGenericRest
+                     : fam == sfmm::kMfmaKernels && n <= sfmm::team_items(op, pb);
     e = sfmm::launch_kernel(op, k, dev_items, n, src_pool, dst_pool, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(ctx, e, "kernel launch");
     return SFMM_OK;

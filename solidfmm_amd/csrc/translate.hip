@@ -160,7 +160,7 @@ hipError_t launch_kernel(int op, const KernelChoice &k, const sfmm_item *items, 
     }
     case kMfmaKernels: {
         const int mode = (!k.acc && k.seg) ? 2 : acc;
-        if (k.compact || n <= team_items(op, k.pk)) return launch_team(op, k.pk, items, n, src, dst, stream, mode);
+        if (k.team) return launch_team(op, k.pk, items, n, src, dst, stream, mode);
         switch (op) {
         case SFMM_M2M: return octet::launch_op<SFMM_M2M>(k.pk, items, n, src, dst, stream, mode);
         case SFMM_M2L: return octet::launch_op<SFMM_M2L>(k.pk, items, n, src, dst, stream, mode);
@@ -172,18 +172,9 @@ hipError_t launch_kernel(int op, const KernelChoice &k, const sfmm_item *items, 
         // as their LDS triangle reaches (M2L, 2,000 items: order 25 340 ->
         // 27 us, 32 577 -> 40, 40 895 -> 84, 48 2500 -> 121; a single group
         // of 7 items: order 32 488 -> 31).
-        if (generic_bucket(k.pk) != kGenericRest) return launch_team(op, k.pk, items, n, src, dst, stream, acc);
+        if (k.team) return launch_team(op, k.pk, items, n, src, dst, stream, acc);
         return launch_generic(op, k.pk, items, n, src, dst, stream, acc);
     }
-}
-
-hipError_t launch_translate(int op, uint32_t p_in, uint32_t p_out, const sfmm_item *items, size_t n,
-                            const double *src, double *dst, hipStream_t stream, int family)
-{
-    if (!have_kernel(op, p_in, p_out, family)) return hipErrorInvalidValue;
-    const uint32_t pb = p_in > p_out ? p_in : p_out;
-    const int fam = family == kAuto ? default_family(pb) : family;
-    return launch_kernel(op, KernelChoice{fam, pb, p_in != p_out}, items, n, src, dst, stream);
 }
 
 }  // namespace sfmm

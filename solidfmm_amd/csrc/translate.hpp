@@ -16,8 +16,9 @@ namespace sfmm {
 //   MFMA     swaps on the FP64 matrix cores, orders up to 24: one wave per
 //            eight translations (octet.hpp, long lists) or several waves per
 //            sixteen (team.hpp);
-//   generic  any orders up to 86: 25 to 48 on the team kernels (team.hpp),
-//            the rest one workgroup per translation (generic.hip).
+//   generic  any orders up to 86, one workgroup per translation
+//            (generic.hip); orders 25 to 48 on the team kernels (team.hpp)
+//            unless the context asks for this family.
 // Lane and octet kernels are instantiated per order bound PB.  Lane kernels
 // take items of orders (PB, PB), their RT variants any p_in, p_out <= PB, as
 // all other kernels do.
@@ -107,7 +108,9 @@ size_t team_items(int op, uint32_t pb);
 
 // Launch bucket of an FP64 item of the generic family, by its larger order:
 // 32 (orders 25 to 32) and kTeamMax (33 to 48) run on team kernels of their
-// own registers and LDS, everything else together on the generic kernel.
+// own registers and LDS, everything else together on the generic kernel (all
+// of them in a context that asks for it: then the team kernels have a path of
+// other steps to be compared with).
 inline constexpr uint32_t kGenericRest = 0;
 uint32_t generic_bucket(uint32_t pb);
 
@@ -126,9 +129,9 @@ struct KernelChoice {
     // scratch mode with runs of one target's items sharing a block (FP64
     // lane, team and octet kernels; the plan lays the runs out)
     bool seg = false;
-    // team kernels for any number of items (their runs are twice as long as
-    // the octet kernels')
-    bool compact = false;
+    // MFMA and generic families: the team kernels, not the octet and generic
+    // ones.  Decided with the runs, which are as long as the kernel's groups.
+    bool team = false;
 };
 
 // Segmented reduction: target block t += sum of its items' scratch blocks,
@@ -165,10 +168,5 @@ hipError_t launch_p2m(const double *pts, const sfmm_cell *cells, size_t n_cells,
                       int dim, hipStream_t stream);
 hipError_t launch_l2p(const double *pts, const sfmm_cell *cells, size_t n_cells, uint32_t max_order,
                       const double *pool, double *phi, double *grad, int dim, hipStream_t stream);
-
-// Enqueue dst += T(src) for n items all of orders (p_in, p_out) with
-// pairwise distinct targets, in `family` (kAuto: default_family).
-hipError_t launch_translate(int op, uint32_t p_in, uint32_t p_out, const sfmm_item *items, size_t n,
-                            const double *src, double *dst, hipStream_t stream, int family = kAuto);
 
 }  // namespace sfmm

@@ -148,3 +148,29 @@ def test_low_orders_mixed(sfmm, orc, op, family):
         err = block_errors(run(sfmm, op, items, src, np.zeros(do), family), want, np.zeros(do), items).max()
         print(f"mixed op {op} family {family} repeats {repeats}: {err:.2e} (tol {tol:.2e})", flush=True)
         assert err <= tol
+
+
+@pytest.mark.parametrize("op", OPS)
+def test_forced_generic_kernel(sfmm, orc, op):
+    """A context that asks for the generic family gets one launch of the
+    one-workgroup kernel for all orders; the default has the team kernels for
+    25 to 32 and for 33 to 48."""
+    parts = [physical_batch(orc, op, P, P, 5, 13 * P + op) for P in (20, 27, 36)]
+    items, src, off = [], [], [0, 0]
+    for it, s, d in parts:
+        it = it.copy()
+        it["src"] += np.uint64(off[0])
+        it["dst"] += np.uint64(off[1])
+        items.append(it)
+        src.append(s)
+        off = [off[0] + len(s), off[1] + len(d)]
+    items, src, zero = np.concatenate(items), np.concatenate(src), np.zeros(off[1])
+    for family, launches in ((0, 3), (3, 1)):
+        ctx = sfmm.Context(36)
+        ctx.set_kernels(family)
+        info = sfmm.Plan(ctx, op, items).launch_info()
+        assert len(info) == launches, info
+    want = orc.translate(op, items, src, zero.copy())
+    naive = orc.translate(op, items, src, zero.copy(), naive=True)
+    tol = max(20 * block_errors(naive, want, zero, items).max(), 1e-13)
+    assert block_errors(run(sfmm, op, items, src, zero, 3), want, zero, items).max() <= tol
