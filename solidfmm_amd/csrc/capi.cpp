@@ -237,8 +237,9 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
     constexpr int kNoKernel = -2, kUnknown = -1;
     std::vector<int8_t> fam_of(size_t(ctx->P + 1) * (ctx->P + 1), int8_t(kUnknown));
     const bool team_generic = generic_on_teams(ctx);
-    const bool small_m2l = op == SFMM_M2L && n <= sfmm::kLaneSmallM2L && ctx->precision == SFMM_FP64 &&
-                           ctx->family == SFMM_KERNELS_AUTO;
+    // neither the context nor its precision fixes the kernels
+    const bool choices_free = ctx->precision == SFMM_FP64 && ctx->family == SFMM_KERNELS_AUTO;
+    const bool small_m2l = op == SFMM_M2L && n <= sfmm::kLaneSmallM2L && choices_free;
     for (size_t i = 0; i < n; ++i) {
         const sfmm_item &it = items[i];
         if (it.p_in > ctx->P || it.p_out > ctx->P)
@@ -274,7 +275,7 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
         for (Key &k : keys) k.round = 0;
     // Long buckets of repeated targets stay on the lane kernels up to
     // kLaneRunsMax, unless the context or its tuning chooses a family.
-    if (plan.scratch && ctx->precision == SFMM_FP64 && ctx->family == SFMM_KERNELS_AUTO) {
+    if (plan.scratch && choices_free) {
         size_t count[sfmm::kLaneRunsMax + 1] = {};
         auto movable = [&](const Key &k) {
             return k.family == sfmm::kMfmaKernels && k.pb <= sfmm::kLaneRunsMax && !ctx->tune[op][k.pb];
@@ -345,20 +346,24 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
         const Key &key = keys[k];
         if (k == 0 || keys[k - 1].round != key.round || keys[k - 1].family != key.family ||
             keys[k - 1].pb != key.pb) {
-            plan.launches.push_back(
-                {{key.family, key.family == sfmm::kGenericKernel ? 0u : key.pb, false, ctx->precision, !plan.scratch},
-                 ordered.size(), 0, key.round});
             size_t count = 1;
             while (k + count < m && keys[k + count].round == key.round && keys[k + count].family == key.family &&
                    keys[k + count].pb == key.pb)
                 ++count;
-            const bool team = key.family == sfmm::kGenericKernel
+            int family = key.family;
+            if (family == sfmm::kMfmaKernels && choices_free && !plan.scratch && !ctx->tune[op][key.pb] &&
+                sfmm::lanes_ahead(op, key.pb, count))
+                family = sfmm::kLaneKernels;
+            const bool team = family == sfmm::kGenericKernel
                                   ? key.pb != sfmm::kGenericRest
                                   : (compact && plan.scratch) || count <= sfmm::team_items(op, key.pb);
-            wave = key.family == sfmm::kLaneKernels ? 64 : team ? 16 : 8;
+            wave = family == sfmm::kLaneKernels ? 64 : team ? 16 : 8;
+            plan.launches.push_back(
+                {{family, family == sfmm::kGenericKernel ? 0u : key.pb, false, ctx->precision, !plan.scratch},
+                 ordered.size(), 0, key.round});
             plan.launches.back().k.team = team;
             plan.launches.back().k.seg =
-                runs && (key.family == sfmm::kLaneKernels || key.family == sfmm::kMfmaKernels);
+                runs && (family == sfmm::kLaneKernels || family == sfmm::kMfmaKernels);
             prev = nullptr;
         }
         sfmm_plan::Launch &L = plan.launches.back();

@@ -43,10 +43,14 @@ int default_family(uint32_t pb)
 // An octet kernel walks a group's degrees in one wave, a team kernel side by
 // side in four or eight: 9 us against 8 for a lone group of order 8, 22
 // against 12 at 16, 42 against 20 at 24. The octet kernel does the same work
-// in fewer cycles, so it takes over once groups fill the chip. M2L, team
-// against octet (us):
-//   order  8: 4,096 8.5, 9.3;   8,192 10.8, 9.8;   120,000 99, 46
-//   order 12: 4,096 11.4, 13.5; 8,192 15.7, 14.6;  120,000 178, 101
+// in fewer cycles, so it takes over once groups fill the chip.  Up to order 13
+// that is where team groups begin to share CUs: 4,096 items are 256 groups of
+// 16, and the next one costs all of them a quarter (order 9, 4,000 items 7.8,
+// 4,200 9.9; octets 7.8 and 7.5, from HBM).  Above, the team's shorter chain
+// carries it further. M2L, team against octet (us):
+//   order  8: 4,000 6.5, 7.1;   5,000 8.1, 7.2;    120,000 99, 46
+//   order 10: 4,000 8.4, 9.2;   5,000 12.2, 9.7;   6,000 12.6, 10.0
+//   order 12: 4,000 10.3, 11.6; 5,000 13.8, 11.8;  120,000 178, 101
 //   order 16: 8,192 22.6, 25.7; 12,288 33.2, 26.4; 120,000 288, 204
 //   order 18: 8,192 27.9, 27.3; 12,288 41.8, 41.8; 120,000 378, 288
 //   order 20: 12,288 45.7, 53.0; 24,000 76.5, 76.1; 120,000 425, 365
@@ -54,14 +58,31 @@ int default_family(uint32_t pb)
 //   order 24: 60,000 299, 344;  120,000 584, 626
 // M2M and L2L keep one operand table instead of two and cross over earlier
 // from order 19 (M2M of order 20: 8,192 29.9, 29.0; 12,288 44.8, 45.5;
-// 16,384 51.8, 46.5; order 24: 16,384 67.8, 68.1; 24,000 96.6, 94.4).
+// 16,384 51.8, 46.5; order 24: 16,384 67.8, 68.1; 24,000 96.6, 94.4).  L2L of
+// orders 8 to 12 as M2L within 5 %.
 size_t team_items(int op, uint32_t pb)
 {
-    if (pb <= 13) return 6144;
+    if (pb <= 13) return 4096;
     if (pb <= 18) return 8192;
     if (op != SFMM_M2L) return 12288;
     if (int(pb) > octet::max_order(op)) return ~size_t(0);
     return pb <= 20 ? 24576 : 32768;
+}
+
+// Octet times go up in steps of 8,192 items, a wave of eight for each SIMD;
+// lanes spread any number of items over theirs.  L2L, whose lane kernels need
+// the fewest registers, is faster on lanes after such a step where few waves
+// are in flight: lanes against octets (us, from HBM)
+//   order  9:  8,256 9.6, 10.2;  12,296 10.7, 11.7; 16,384 11.9, 13.0; 16,904 16.5, 16.6
+//             20,000 17.6, 17.5; 25,096 19.0, 20.9; 32,768 22.0, 22.8; 40,000 29.2, 27.2
+//   order 10:  8,256 11.7, 11.8; 12,296 12.9, 13.3; 16,384 14.3, 14.7; 18,000 20.8, 19.9
+//   order 11:  8,256 13.3, 13.9; 12,296 14.7, 15.2; 16,384 16.5, 17.1; 18,000 23.9, 23.1
+// and M2M and M2L of order 9 at 12,000 items: 11.7, 11.5 and 12.0, 10.9.
+bool lanes_ahead(int op, uint32_t pb, size_t n)
+{
+    constexpr size_t step = 8192;
+    if (op != SFMM_L2L || pb < 9 || pb > 11) return false;
+    return (n > step && n <= 2 * step) || (pb == 9 && n > 3 * step && n <= 4 * step);
 }
 
 uint32_t generic_bucket(uint32_t pb)

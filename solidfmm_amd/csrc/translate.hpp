@@ -106,6 +106,9 @@ hipError_t launch_op(uint32_t pb, const sfmm_item *items, size_t n, const double
 // kernel instead of the octet kernel (translate.hip has the figures).
 size_t team_items(int op, uint32_t pb);
 
+// Lists of n items of distinct targets that stay on lanes above kLaneAutoMax.
+bool lanes_ahead(int op, uint32_t pb, size_t n);
+
 // Launch bucket of an FP64 item of the generic family, by its larger order:
 // 32 (orders 25 to 32) and kTeamMax (33 to 48) run on team kernels of their
 // own registers and LDS, everything else together on the generic kernel (all
