@@ -26,7 +26,7 @@ COMMON = [
 
 # Translation units; the kernel instantiations are split so they compile in
 # parallel, the longest first.
-SOURCES = ["octet_m2l.hip", "octet_m2m.hip", "octet_l2l.hip", "team_m2l.hip", "team_m2m.hip", "team_l2l.hip", "mfma_prec_hi.hip", "mfma_prec_mid.hip", "lane_prec_dw.hip", "lane_prec_f32.hip", "lane_rt.hip", "lane_fixed.hip", "prec_generic.hip", "mfma_prec.hip", "reduce.hip", "particles.hip", "translate.hip", "team.hip", "generic.hip", "arith_probe.hip", "swap_host.cpp", "capi.cpp", "dropin.cpp",
+SOURCES = ["octet_m2l.hip", "octet_m2m.hip", "octet_l2l.hip", "team_m2l.hip", "team_m2m.hip", "team_l2l.hip", "mfma_prec_hi.hip", "mfma_prec_mid.hip", "lane_prec_dw.hip", "lane_prec_f32.hip", "lane_runs.hip", "lane_rt.hip", "lane_fixed.hip", "prec_generic.hip", "mfma_prec.hip", "reduce.hip", "particles.hip", "translate.hip", "team.hip", "generic.hip", "arith_probe.hip", "swap_host.cpp", "capi.cpp", "dropin.cpp",
            "sphere.cpp", "server.cpp"]
 
 # Host-only C++ (the drop-in API over the C ABI).

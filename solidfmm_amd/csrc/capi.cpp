@@ -342,6 +342,7 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
     const sfmm_item *prev = nullptr;
     uint64_t run_off = 0;
     size_t wave = 64;  // items a run of the launch may span
+    size_t heads = 0;  // runs of the launch so far
     for (size_t k = 0; k < m; ++k) {
         const Key &key = keys[k];
         if (k == 0 || keys[k - 1].round != key.round || keys[k - 1].family != key.family ||
@@ -365,6 +366,7 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
             plan.launches.back().k.seg =
                 runs && (family == sfmm::kLaneKernels || family == sfmm::kMfmaKernels);
             prev = nullptr;
+            heads = 0;
         }
         sfmm_plan::Launch &L = plan.launches.back();
         if (key.family == sfmm::kGenericKernel) {
@@ -378,6 +380,7 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
             const bool join = L.k.seg && prev && L.count % wave != 0 && prev->dst == src_it.dst &&
                               prev->p_in == src_it.p_in && prev->p_out == src_it.p_out && !zero(*prev) &&
                               !zero(src_it);
+            heads += !join;
             if (!join) {  // a block of its own in the scratch pool
                 run_off = scratch_reals;
                 scratch_reals += size_t(it.p_out) * (it.p_out + 1);
@@ -390,6 +393,7 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
         prev = &src_it;
         ordered.push_back(it);
         L.count++;
+        L.k.long_runs = L.k.seg && L.k.family == sfmm::kLaneKernels && sfmm::long_runs(L.k.pk, L.count, heads);
     }
     // Reduction tables: targets in order of first appearance, each with its
     // scratch blocks in the list order of their first items (a run's block

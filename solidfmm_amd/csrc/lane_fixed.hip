@@ -9,7 +9,7 @@ namespace lane {
 
 const Table &fixed_table()
 {
-    static const Table t = make_table<false>();
+    static const Table t = make_table<false, false>();
     return t;
 }
 

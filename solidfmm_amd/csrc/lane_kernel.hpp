@@ -30,6 +30,8 @@
 //               >= p_out are not stored.  Degrees above the largest order
 //               of the wave are skipped with wave-uniform branches, so a
 //               wave of equal orders does the work of its own orders.
+//               With SUMS, for lists whose targets repeat in long runs, a
+//               wave of few runs adds them through LDS (run_sums).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -237,10 +239,9 @@ struct Segments {
     bool head = true;    // this lane stores its run's sum
     uint64_t heads = 0;  // first lanes of the wave's runs where it has few (run_sums)
 };
-// Waves of at most this many runs add them through LDS.  The tree of
-// shuffles costs the same for any runs, the LDS sums some 15 instructions a
-// run and degree: equal at about 16.
-inline constexpr int kFewRuns = 8;
+// Waves of at most this many runs add them through LDS where the kernel has
+// that (long_runs).
+inline constexpr int kFewRuns = 5;
 // doubles per lane of the LDS copy of one degree (odd: no bank conflicts),
 // and beyond the last lane
 template <int P>
@@ -357,16 +358,17 @@ inline constexpr int kLaneWaves = (PI == 7 || PI == 8) ? 2 : 1;
 // first ipw lanes; a launch sized below a whole number of rounds of resident
 // waves spreads its items evenly over one more round instead of leaving
 // that round's waves partly empty (launch_kernel).
-template <int OP, int PI, int PO, bool RT>
+template <int OP, int PI, int PO, bool RT, bool SUMS>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kLaneWaves<OP, PI>)))
     k_translate(const double *__restrict__ src_pool, double *__restrict__ dst_pool,
                 const sfmm_item *__restrict__ items, uint32_t n_items, int acc, uint32_t ipw)
 {
     static_assert(!RT || PI == PO, "runtime orders use a square bound");
+    static_assert(RT || !SUMS, "runs come with runtime orders");
     constexpr int PM = PI > PO ? PI : PO;
     constexpr int PE = PI < PO ? PI : PO;
     // a degree of the wave's results, for run_sums
-    __shared__ double sums[RT ? 64 * kSumStride<PI> + kSumPad : 1];
+    __shared__ double sums[SUMS ? 64 * kSumStride<PI> + kSumPad : 1];
     const uint32_t lane_id = threadIdx.x;
     const uint32_t t = lane_id < ipw ? blockIdx.x * ipw + lane_id : n_items;
     // runs (acc == 2) exist in the per-item-order kernels only; the plan
@@ -403,7 +405,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kLaneWa
         y = -y;
         z = -z;
     }
-    if constexpr (RT) {
+    if constexpr (SUMS) {
         const uint64_t heads = __ballot(seg.head);
         if (acc == 2 && __ballot(true) == ~uint64_t(0) && __popcll(heads) <= kFewRuns) seg.heads = heads;
     }
@@ -419,9 +421,11 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kLaneWa
         constexpr int N = decltype(Nc)::value;
         if constexpr (RT) {
             if (acc == 2) {
-                if (seg.heads) {
-                    run_sums<N, kSumStride<PI>>(seg, sums, D, re, im, on);
-                    return;
+                if constexpr (SUMS) {
+                    if (seg.heads) {
+                        run_sums<N, kSumStride<PI>>(seg, sums, D, re, im, on);
+                        return;
+                    }
                 }
                 segment_sum<N>(seg, re, im);
                 on = on && seg.head;
@@ -684,25 +688,26 @@ struct Table {
     kernel_fn f[3][kSquare];
 };
 
-template <bool RT, int OP, int... Ps>
+template <bool RT, bool SUMS, int OP, int... Ps>
 constexpr void fill(kernel_fn *tab, std::integer_sequence<int, Ps...>)
 {
-    ((tab[Ps] = &k_translate<OP, Ps + 1, Ps + 1, RT>), ...);
+    ((tab[Ps] = &k_translate<OP, Ps + 1, Ps + 1, RT, SUMS>), ...);
 }
 
-template <bool RT>
+template <bool RT, bool SUMS>
 Table make_table()
 {
     Table t{};
-    fill<RT, SFMM_M2M>(t.f[0], std::make_integer_sequence<int, kSquare>{});
-    fill<RT, SFMM_M2L>(t.f[1], std::make_integer_sequence<int, kSquare>{});
-    fill<RT, SFMM_L2L>(t.f[2], std::make_integer_sequence<int, kSquare>{});
+    fill<RT, SUMS, SFMM_M2M>(t.f[0], std::make_integer_sequence<int, kSquare>{});
+    fill<RT, SUMS, SFMM_M2L>(t.f[1], std::make_integer_sequence<int, kSquare>{});
+    fill<RT, SUMS, SFMM_L2L>(t.f[2], std::make_integer_sequence<int, kSquare>{});
     return t;
 }
 
-// Tables of the two variants (lane_fixed.hip, lane_rt.hip).
+// Tables of the variants (lane_fixed.hip, lane_rt.hip, lane_runs.hip).
 const Table &fixed_table();
 const Table &rt_table();
+const Table &runs_table();
 
 }  // namespace lane
 }  // namespace sfmm

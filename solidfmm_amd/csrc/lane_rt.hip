@@ -9,7 +9,7 @@ namespace lane {
 
 const Table &rt_table()
 {
-    static const Table t = make_table<true>();
+    static const Table t = make_table<true, false>();
     return t;
 }
 

@@ -69,6 +69,18 @@ size_t team_items(int op, uint32_t pb)
     return pb <= 20 ? 24576 : 32768;
 }
 
+// The tree of shuffles costs the same for any runs, the sums through LDS some
+// 15 instructions a run and degree and an LDS copy of the wave's results.  M2L
+// with its reduction, tree against LDS (us), by items and length of the runs:
+//   order  6, 250,000: 16 52, 49; 20 51, 51; 32 50, 42; 140 47, 41
+//   order  8, 250,000: 16 98, 83; 32 92, 74; 140 89, 70;  50,000: 32, 31 at any
+//   order 10, 250,000: 16 180, 151; 140 171, 122;  20,000: 35, 37 at any
+// and at 200,000 items in runs of 8: order 6 50, 65; 9 128, 156; 11 220, 236.
+bool long_runs(uint32_t pb, size_t n, size_t runs)
+{
+    return n >= 65536 && n >= (pb >= 7 ? 16 : 24) * runs;
+}
+
 // Octet times go up in steps of 8,192 items, a wave of eight for each SIMD;
 // lanes spread any number of items over theirs.  L2L, whose lane kernels need
 // the fewest registers, is faster on lanes after such a step where few waves
@@ -169,7 +181,9 @@ hipError_t launch_kernel(int op, const KernelChoice &k, const sfmm_item *items, 
         // scratch launches with runs use the per-item-order kernels (the
         // fixed-order ones have no code for runs)
         const bool runs = !k.acc && k.seg;
-        const lane::Table &t = (k.rt || runs) ? lane::rt_table() : lane::fixed_table();
+        const lane::Table &t = k.long_runs     ? lane::runs_table()
+                               : k.rt || runs ? lane::rt_table()
+                                              : lane::fixed_table();
         lane::kernel_fn f = t.f[op][k.pk - 1];
         const uint32_t block = 64;
         uint32_t ipw = lane_items_per_wave(reinterpret_cast<const void *>(f), n);

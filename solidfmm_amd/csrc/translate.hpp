@@ -40,6 +40,10 @@ inline constexpr uint32_t kLaneAutoMax = 7;
 inline constexpr uint32_t kLaneRunsMax = kLaneMax;
 inline constexpr size_t kLaneRunsItems = 40000;
 
+// Whether a lane launch of n items in `runs` runs adds them through LDS
+// (run_sums) instead of by a tree of shuffles (translate.hip has the figures).
+bool long_runs(uint32_t pb, size_t n, size_t runs);
+
 // M2L lists of at most kLaneSmallM2L items keep orders 9 to 11 on lanes by
 // default.  Small batches are where single results are compared with the
 // reference, and the lanes' sums follow its order: 256 items of order 10
@@ -132,6 +136,8 @@ struct KernelChoice {
     // scratch mode with runs of one target's items sharing a block (FP64
     // lane, team and octet kernels; the plan lays the runs out)
     bool seg = false;
+    // lane kernels: the runs are long_runs
+    bool long_runs = false;
     // MFMA and generic families: the team kernels, not the octet and generic
     // ones.  Decided with the runs, which are as long as the kernel's groups.
     bool team = false;

@@ -61,3 +61,18 @@ def test_default_on_repeated_targets(sfmm, orc, P, n):
     parts = [repeated(orc, W.M2L, P, P, 300, [50], P), repeated(orc, W.M2L, 1, P, n - 300, [90], P + 1)]
     items, src, nd = join(parts)
     check(sfmm, orc, W.M2L, items, src, nd, AUTO, f"default P={P} n={n}")
+
+
+# Lists long enough for the sums through LDS: waves of one run, of a few, and
+# of more than the LDS sums take; runs across waves; a last wave that is not full
+@pytest.mark.parametrize("op", [W.M2M, W.M2L, W.L2L])
+@pytest.mark.parametrize("P", [1, 3, 7, 8, 9, 12])
+def test_long_lists_of_long_runs(sfmm, orc, op, P):
+    parts = [repeated(orc, op, P, P, 64 * 4 + 21, lengths, 5 * P + op)
+             for lengths in ([64], [20], [13, 12, 13], [3, 1, 40, 2, 100, 2])]
+    parts += [repeated(orc, op, 1, P, 66000, [64], P)]
+    items, src, nd = join(parts)
+    if op != W.M2L:
+        for c in "xyz":
+            items[c][130:200:13] = 0.0
+    check(sfmm, orc, op, items, src, nd, LANE, f"op {op} P={P}")
