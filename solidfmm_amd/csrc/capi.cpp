@@ -273,18 +273,6 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
     plan.scratch = rounds > kMaxRounds;
     if (plan.scratch)
         for (Key &k : keys) k.round = 0;
-    // Long buckets of repeated targets stay on the lane kernels up to
-    // kLaneRunsMax, unless the context or its tuning chooses a family.
-    if (plan.scratch && choices_free) {
-        size_t count[sfmm::kLaneRunsMax + 1] = {};
-        auto movable = [&](const Key &k) {
-            return k.family == sfmm::kMfmaKernels && k.pb <= sfmm::kLaneRunsMax && !ctx->tune[op][k.pb];
-        };
-        for (const Key &k : keys)
-            if (movable(k)) ++count[k.pb];
-        for (Key &k : keys)
-            if (movable(k) && count[k.pb] > sfmm::kLaneRunsItems) k.family = sfmm::kLaneKernels;
-    }
     // keys are in list order here: remember each item's position in it
     std::vector<uint32_t> list_pos;
     if (plan.scratch) {
@@ -336,64 +324,64 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
     // among the items of a run: consecutive items of a launch, within one
     // 64-item wave (lane kernels) or group of 8 (octet kernels) or 16 (team
     // kernels), with the same target and orders and a nonzero shift (the
-    // kernels add a run's results across lanes).
+    // kernels add a run's results across lanes).  follows[k]: item k can join
+    // the run of item k - 1.
     const bool runs = plan.scratch && ctx->precision == SFMM_FP64;
     auto zero = [](const sfmm_item &it) { return it.x == 0.0 && it.y == 0.0 && it.z == 0.0; };
-    const sfmm_item *prev = nullptr;
+    std::vector<uint8_t> follows(runs ? m : 0);
     uint64_t run_off = 0;
-    size_t wave = 64;  // items a run of the launch may span
-    size_t heads = 0;  // runs of the launch so far
-    for (size_t k = 0; k < m; ++k) {
-        const Key &key = keys[k];
-        if (k == 0 || keys[k - 1].round != key.round || keys[k - 1].family != key.family ||
-            keys[k - 1].pb != key.pb) {
-            size_t count = 1;
-            while (k + count < m && keys[k + count].round == key.round && keys[k + count].family == key.family &&
-                   keys[k + count].pb == key.pb)
-                ++count;
-            int family = key.family;
-            if (family == sfmm::kMfmaKernels && choices_free && !plan.scratch && !ctx->tune[op][key.pb] &&
-                sfmm::lanes_ahead(op, key.pb, count))
-                family = sfmm::kLaneKernels;
-            const bool team = family == sfmm::kGenericKernel
-                                  ? key.pb != sfmm::kGenericRest
-                                  : (compact && plan.scratch) || count <= sfmm::team_items(op, key.pb);
-            wave = family == sfmm::kLaneKernels ? 64 : team ? 16 : 8;
-            plan.launches.push_back(
-                {{family, family == sfmm::kGenericKernel ? 0u : key.pb, false, ctx->precision, !plan.scratch},
-                 ordered.size(), 0, key.round});
-            plan.launches.back().k.team = team;
-            plan.launches.back().k.seg =
-                runs && (family == sfmm::kLaneKernels || family == sfmm::kMfmaKernels);
-            prev = nullptr;
-            heads = 0;
-        }
-        sfmm_plan::Launch &L = plan.launches.back();
-        if (key.family == sfmm::kGenericKernel) {
-            L.k.pk = std::max({L.k.pk, key.p_in, key.p_out});
-        } else if (key.p_in != key.pb || key.p_out != key.pb) {
-            L.k.rt = true;
-        }
-        const sfmm_item &src_it = items[key.index];
-        sfmm_item it = src_it;
-        if (plan.scratch) {
-            const bool join = L.k.seg && prev && L.count % wave != 0 && prev->dst == src_it.dst &&
-                              prev->p_in == src_it.p_in && prev->p_out == src_it.p_out && !zero(*prev) &&
-                              !zero(src_it);
-            heads += !join;
-            if (!join) {  // a block of its own in the scratch pool
-                run_off = scratch_reals;
-                scratch_reals += size_t(it.p_out) * (it.p_out + 1);
-            } else {
-                is_head[list_pos[key.index]] = 0;
+    for (size_t begin = 0, end; begin < m; begin = end) {
+        const Key &first = keys[begin];
+        for (end = begin + 1; end < m && keys[end].round == first.round && keys[end].family == first.family &&
+                              keys[end].pb == first.pb;)
+            ++end;
+        const size_t count = end - begin;
+        const bool seg = runs && (first.family == sfmm::kLaneKernels || first.family == sfmm::kMfmaKernels);
+        size_t lane_runs = 0;  // runs within 64 items
+        for (size_t k = begin; seg && k < end; ++k) {
+            if (k > begin) {
+                const sfmm_item &a = items[keys[k - 1].index], &b = items[keys[k].index];
+                follows[k] = a.dst == b.dst && a.p_in == b.p_in && a.p_out == b.p_out && !zero(a) && !zero(b);
             }
-            scr_off[list_pos[key.index]] = run_off;
-            it.dst = run_off;
+            lane_runs += !(follows[k] && (k - begin) % 64 != 0);
         }
-        prev = &src_it;
-        ordered.push_back(it);
-        L.count++;
-        L.k.long_runs = L.k.seg && L.k.family == sfmm::kLaneKernels && sfmm::long_runs(L.k.pk, L.count, heads);
+        int family = first.family;
+        if (family == sfmm::kMfmaKernels && choices_free && !ctx->tune[op][first.pb] &&
+            (seg ? sfmm::lanes_for_runs(op, first.pb, count, lane_runs, m) : sfmm::lanes_ahead(op, first.pb, count)))
+            family = sfmm::kLaneKernels;
+        const bool lanes = family == sfmm::kLaneKernels;
+        const bool team = family == sfmm::kGenericKernel
+                              ? first.pb != sfmm::kGenericRest
+                              : (compact && plan.scratch) || count <= sfmm::team_items(op, first.pb);
+        const size_t wave = lanes ? 64 : team ? 16 : 8;  // items a run may span
+        plan.launches.push_back(
+            {{family, family == sfmm::kGenericKernel ? 0u : first.pb, false, ctx->precision, !plan.scratch},
+             ordered.size(), count, first.round});
+        sfmm::KernelChoice &choice = plan.launches.back().k;
+        choice.seg = seg;
+        choice.team = team;
+        choice.long_runs = seg && lanes && sfmm::long_runs(first.pb, count, lane_runs);
+        for (size_t k = begin; k < end; ++k) {
+            const Key &key = keys[k];
+            if (family == sfmm::kGenericKernel) {
+                choice.pk = std::max({choice.pk, key.p_in, key.p_out});
+            } else if (key.p_in != key.pb || key.p_out != key.pb) {
+                choice.rt = true;
+            }
+            sfmm_item it = items[key.index];
+            if (plan.scratch) {
+                const uint32_t pos = list_pos[key.index];
+                if (!seg || !follows[k] || (k - begin) % wave == 0) {  // a block of its own in the scratch pool
+                    run_off = scratch_reals;
+                    scratch_reals += size_t(it.p_out) * (it.p_out + 1);
+                } else {
+                    is_head[pos] = 0;
+                }
+                scr_off[pos] = run_off;
+                it.dst = run_off;
+            }
+            ordered.push_back(it);
+        }
     }
     // Reduction tables: targets in order of first appearance, each with its
     // scratch blocks in the list order of their first items (a run's block

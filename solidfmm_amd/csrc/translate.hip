@@ -97,6 +97,49 @@ bool lanes_ahead(int op, uint32_t pb, size_t n)
     return (n > step && n <= 2 * step) || (pb == 9 && n > 3 * step && n <= 4 * step);
 }
 
+// A lane wave adds runs of up to 64 items before it stores, an octet group runs
+// of up to 8, and a lane takes one translation's latency for 64 of them; but 64
+// items a wave need long lists to fill the chip.  The lists from which lanes are
+// ahead, by order and by mean length of the runs; M2L with its reduction, lanes
+// against octets (us) by items and length:
+//   order  8: 100,000  5 60, 58;   16 45, 50;   140 42, 51;  500,000  5 220, 258; 140 113, 204
+//   order  9: 100,000 20 67, 62;   32 58, 62;   200,000 16 105, 113;  500,000  5 284, 313
+//   order 10: 100,000 32 74, 73;   64 71, 72;   200,000 16 126, 136;  500,000 12 320, 321
+//   order 11: 300,000 16 239, 228; 32 215, 226; 200,000 140 129, 154; 500,000 12 431, 376
+//   order 12: 300,000 64 271, 248; 140 236, 254; 500,000 140 342, 408; 200,000 140 176, 175
+// M2M, whose runs are the up to eight children of a cell: order 8, 500,000
+// 238, 248; order 9 300,000 177, 186; order 12 616, 478.  The lane kernels of
+// L2L are slower at any length (order 8, 500,000: 5 395, 274; 140 287, 215).
+// One round of lane waves, 65,536 items, takes the same time from 40,000 on:
+// M2L of order 9, 60,000: 16 37, 43; order 10: 16 45, 50; order 11: 140 54, 60;
+// and two waves fit a SIMD at order 8, 130,000: 5 69, 72; 12 58, 63.
+//
+// Launches of one plan run side by side and fill each other's last rounds, so
+// what counts is the plan's `total`, as long as the launch itself has work for
+// most SIMDs: M2L of an FMM, 75,000 of its 997,000 items of order 11, 823 us
+// with that bucket on lanes, 847 on octets; 30,000 of order 12 869 and 847.
+bool lanes_for_runs(int op, uint32_t pb, size_t n, size_t runs, size_t total)
+{
+    constexpr size_t no = ~size_t(0);
+    struct Row {
+        size_t len4, len16, len24, len40;  // items from which lanes are ahead
+        size_t round, full, round_len;     // one round of M2L: items from, to, length
+    };
+    constexpr Row rows[] = {{200000, 100000, 100000, 70000, 110000, 131072, 4},
+                            {300000, 200000, 100000, 100000, 43000, 65536, 10},
+                            {450000, 200000, 150000, 100000, 48000, 65536, 16},
+                            {no, 500000, 250000, 150000, 57000, 65536, 40},
+                            {no, no, no, 300000, no, 0, 0}};
+    if (op == SFMM_L2L || pb < 8 || pb > kLaneMax || n <= 40000) return false;
+    const Row &r = rows[pb - 8];
+    if (op == SFMM_M2L && total == n && n >= r.round && n <= r.full && n >= r.round_len * runs) return true;
+    return total >= (n >= 40 * runs   ? r.len40
+                     : n >= 24 * runs ? r.len24
+                     : n >= 16 * runs ? r.len16
+                     : n >= 4 * runs  ? r.len4
+                                      : no);
+}
+
 uint32_t generic_bucket(uint32_t pb)
 {
     if (pb <= uint32_t(mfma::kMfmaMax) || pb > kTeamMax) return kGenericRest;

@@ -31,15 +31,6 @@ inline constexpr uint32_t kLaneMax = 12;
 // 211, 149), and on short lists of order 8 behind the team kernels (1,000:
 // 11.9 against 8.1; order 7, 4,000: 8.2, 8.4)
 inline constexpr uint32_t kLaneAutoMax = 7;
-// ... and up to this one on lists of repeated targets with more than
-// kLaneRunsItems items: a lane wave adds runs of up to 64 items before it
-// stores, an octet group runs of up to 8, but 64 items a wave need long lists
-// to fill the chip.  Interaction lists of grids, M2L with its reduction, lanes
-// against octets (us): order 8, 29,078 items 26.1, 23.2; 53,352 29.2, 32.7;
-// 374,976 79, 150; order 12 49.9, 43.4; 56.0, 61.2; 232, 302.
-inline constexpr uint32_t kLaneRunsMax = kLaneMax;
-inline constexpr size_t kLaneRunsItems = 40000;
-
 // Whether a lane launch of n items in `runs` runs adds them through LDS
 // (run_sums) instead of by a tree of shuffles (translate.hip has the figures).
 bool long_runs(uint32_t pb, size_t n, size_t runs);
@@ -110,8 +101,11 @@ hipError_t launch_op(uint32_t pb, const sfmm_item *items, size_t n, const double
 // kernel instead of the octet kernel (translate.hip has the figures).
 size_t team_items(int op, uint32_t pb);
 
-// Lists of n items of distinct targets that stay on lanes above kLaneAutoMax.
+// Launches above kLaneAutoMax that stay on lanes: n items of distinct targets,
+// and n of the `total` items of a plan of repeated targets that are `runs` runs
+// in lane waves.
 bool lanes_ahead(int op, uint32_t pb, size_t n);
+bool lanes_for_runs(int op, uint32_t pb, size_t n, size_t runs, size_t total);
 
 // Launch bucket of an FP64 item of the generic family, by its larger order:
 // 32 (orders 25 to 32) and kTeamMax (33 to 48) run on team kernels of their

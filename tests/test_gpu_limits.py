@@ -48,3 +48,18 @@ def test_l2l_default(sfmm, orc, P, n, family):
     naive = orc.translate(W.L2L, few, src, zero.copy(), naive=True)
     tol = max(20 * block_errors(naive, want, zero, few).max(), 1e-13)
     assert block_errors(d.cpu().numpy(), want, zero, items).max() <= tol
+
+
+# Repeated targets: lanes for long lists of long runs, by their mean length
+# and not by the one target that repeats most
+@pytest.mark.parametrize("op,P,n,lengths,family", [
+    (W.M2L, 12, 70000, [5] + [1] * 69995, MFMA),   # one target of five items
+    (W.M2L, 12, 70000, [40], MFMA), (W.M2M, 10, 70000, [8], MFMA), (W.L2L, 8, 110000, [64], MFMA),
+    (W.M2L, 8, 110000, [64], LANE), (W.M2M, 9, 110000, [40], LANE), (W.M2L, 9, 50000, [64], LANE),
+    (W.M2L, 9, 66000, [20], MFMA), (W.M2M, 9, 50000, [64], MFMA), (W.M2L, 11, 110000, [64], MFMA)])
+def test_repeated_targets_default(sfmm, orc, op, P, n, lengths, family):
+    parts = [repeated(orc, op, P, P, 50, [16, 17, 3], P), repeated(orc, op, 1, P, n - 50, lengths, P + 1)]
+    items, src, nd = join(parts)
+    info = sfmm.Plan(sfmm.Context(P), op, items).launch_info()
+    assert [i[0] for i in info] == [family], info
+    check(sfmm, orc, op, items, src, nd, AUTO, f"op {op} P={P} n={n}")
