@@ -231,6 +231,7 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
     std::vector<Key> keys;
     keys.reserve(n);
     FlatMap seen;  // target -> occurrences so far
+    size_t src_begin = ~size_t(0), src_read = 0;  // first source, reals read
     uint32_t rounds = 0;
     // kernel family per (p_in, p_out), filled on first use: lists repeat a
     // handful of order pairs millions of times
@@ -262,7 +263,10 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
         bool fresh;
         const uint32_t round = seen.get(it.dst, 0, fresh)++;
         rounds = std::max(rounds, round + 1);
-        plan.src_extent = std::max<size_t>(plan.src_extent, it.src + size_t(it.p_in) * (it.p_in + 1));
+        const size_t src_end = it.src + size_t(it.p_in) * (it.p_in + 1);
+        plan.src_extent = std::max(plan.src_extent, src_end);
+        src_begin = std::min<size_t>(src_begin, it.src);
+        src_read += src_end - it.src;
         plan.dst_extent = std::max<size_t>(plan.dst_extent, it.dst + size_t(it.p_out) * (it.p_out + 1));
         // the generic kernels take many orders in one launch
         uint32_t bucket = pb;
@@ -270,6 +274,7 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
             bucket = team_generic ? sfmm::generic_bucket(pb) : sfmm::kGenericRest;
         keys.push_back({round, fam, bucket, it.p_in, it.p_out, i});
     }
+    const bool shared = !keys.empty() && src_read >= 2 * (plan.src_extent - src_begin);
     plan.scratch = rounds > kMaxRounds;
     if (plan.scratch)
         for (Key &k : keys) k.round = 0;
@@ -347,7 +352,7 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
         }
         int family = first.family;
         if (family == sfmm::kMfmaKernels && choices_free && !ctx->tune[op][first.pb] &&
-            (seg ? sfmm::lanes_for_runs(op, first.pb, count, lane_runs, m) : sfmm::lanes_ahead(op, first.pb, count)))
+            (seg ? sfmm::lanes_for_runs(op, first.pb, count, lane_runs, m) : sfmm::lanes_ahead(op, first.pb, count, shared)))
             family = sfmm::kLaneKernels;
         const bool lanes = family == sfmm::kLaneKernels;
         const bool team = family == sfmm::kGenericKernel

@@ -90,11 +90,16 @@ bool long_runs(uint32_t pb, size_t n, size_t runs)
 //   order 10:  8,256 11.7, 11.8; 12,296 12.9, 13.3; 16,384 14.3, 14.7; 18,000 20.8, 19.9
 //   order 11:  8,256 13.3, 13.9; 12,296 14.7, 15.2; 16,384 16.5, 17.1; 18,000 23.9, 23.1
 // and M2M and M2L of order 9 at 12,000 items: 11.7, 11.5 and 12.0, 10.9.
-bool lanes_ahead(int op, uint32_t pb, size_t n)
+// Children that share their parent's expansion read it from the caches, and the
+// lanes' single accesses cost less: lanes ahead at any length from there on, with
+// the pools in HBM (8 children; order 9 12,000 9.5, 10.7; 100,000 56, 61; 300,000
+// 157, 178; order 10 12,000 11.4, 12.5; 200,000 136, 140; order 11 25,000 21.7,
+// 24.9; 300,000 230, 245) as in the last-level cache (order 10, 100,000 47, 60).
+bool lanes_ahead(int op, uint32_t pb, size_t n, bool shared)
 {
     constexpr size_t step = 8192;
     if (op != SFMM_L2L || pb < 9 || pb > 11) return false;
-    return (n > step && n <= 2 * step) || (pb == 9 && n > 3 * step && n <= 4 * step);
+    return n > step && (shared || n <= 2 * step || (pb == 9 && n > 3 * step && n <= 4 * step));
 }
 
 // A lane wave adds runs of up to 64 items before it stores, an octet group runs

@@ -101,10 +101,10 @@ hipError_t launch_op(uint32_t pb, const sfmm_item *items, size_t n, const double
 // kernel instead of the octet kernel (translate.hip has the figures).
 size_t team_items(int op, uint32_t pb);
 
-// Launches above kLaneAutoMax that stay on lanes: n items of distinct targets,
-// and n of the `total` items of a plan of repeated targets that are `runs` runs
+// Launches above kLaneAutoMax that stay on lanes: n items of distinct targets
+// (shared: whose list reads a source twice or more on average), and n of the `total` items of a plan of repeated targets that are `runs` runs
 // in lane waves.
-bool lanes_ahead(int op, uint32_t pb, size_t n);
+bool lanes_ahead(int op, uint32_t pb, size_t n, bool shared);
 bool lanes_for_runs(int op, uint32_t pb, size_t n, size_t runs, size_t total);
 
 // Launch bucket of an FP64 item of the generic family, by its larger order:

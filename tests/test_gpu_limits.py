@@ -63,3 +63,22 @@ def test_repeated_targets_default(sfmm, orc, op, P, n, lengths, family):
     info = sfmm.Plan(sfmm.Context(P), op, items).launch_info()
     assert [i[0] for i in info] == [family], info
     check(sfmm, orc, op, items, src, nd, AUTO, f"op {op} P={P} n={n}")
+
+
+@pytest.mark.parametrize("P,n,family", [(9, 8192, MFMA), (9, 20000, LANE), (10, 30000, LANE), (11, 17000, LANE),
+                                        (8, 20000, MFMA), (12, 20000, MFMA)])
+def test_l2l_of_children_default(sfmm, orc, P, n, family):
+    """L2L from parents of eight children, orders 9 to 11, stays on lanes."""
+    items, src, dst = physical_batch(orc, W.L2L, P, P, n, P + n)
+    items["src"] = items["src"][np.arange(n) // 8]
+    ctx = sfmm.Context(P)
+    plan = sfmm.Plan(ctx, W.L2L, items)
+    assert [i[0] for i in plan.launch_info()] == [family]
+    zero = np.zeros(len(dst))
+    d = torch.zeros(len(dst), dtype=torch.float64, device="cuda")
+    plan.execute(torch.from_numpy(src).to("cuda"), d)
+    torch.cuda.synchronize()
+    want = orc.translate(W.L2L, items, src, zero.copy())
+    naive = orc.translate(W.L2L, items[:200], src, zero.copy(), naive=True)
+    tol = max(20 * block_errors(naive, want, zero, items[:200]).max(), 1e-13)
+    assert block_errors(d.cpu().numpy(), want, zero, items).max() <= tol
