@@ -139,6 +139,12 @@ int sfmm_plan_create(sfmm_context *ctx, int op, const sfmm_item *host_items, siz
  * the copy), and keep `dev_mem` to the plan until its last launch has
  * completed. */
 int sfmm_plan_prepare(sfmm_context *ctx, int op, const sfmm_item *host_items, size_t n, sfmm_plan **plan);
+/* The same for an arena of `max_bytes`: a list of repeated targets whose plan
+ * would need more takes kernels that share scratch blocks among more items, if
+ * it fits with those (results agree to rounding), and is the plan of
+ * sfmm_plan_prepare otherwise. */
+int sfmm_plan_prepare_within(sfmm_context *ctx, int op, const sfmm_item *host_items, size_t n, size_t max_bytes,
+                             sfmm_plan **plan);
 size_t sfmm_plan_device_bytes(const sfmm_plan *plan);
 int sfmm_plan_bind(sfmm_plan *plan, void *dev_mem, size_t dev_bytes, void *stream);
 /* As sfmm_plan_bind, but the tables go through caller-owned pinned host
@@ -305,7 +311,7 @@ int sfmm_device(const sfmm_context *ctx);
  * runs requests on `slots` streams of its own:
  *   - sfmm_server_submit copies a request (operator, items, the cells it
  *     reads and writes) and queues it in arrival order; `workers` host
- *     threads prepare plans (sfmm_plan_prepare) while the GPU runs others,
+ *     threads prepare plans (sfmm_plan_prepare_within) while the GPU runs others,
  *     at a lower CPU priority (niceness 5) than the server's scheduling
  *     thread, which should have a core to itself;
  *   - the oldest waiting request is admitted when it is prepared, a slot is

@@ -50,6 +50,7 @@ SIGNATURES = {
     "sfmm_plan_create": (_c.c_int, [_vp, _c.c_int, _vp, _c.c_size_t, _c.POINTER(_vp)]),
     "sfmm_plan_prepare": (_c.c_int, [_vp, _c.c_int, _vp, _c.c_size_t, _c.POINTER(_vp)]),
     "sfmm_plan_bind": (_c.c_int, [_vp, _vp, _c.c_size_t, _vp]),
+    "sfmm_plan_prepare_within": (_c.c_int, [_vp, _c.c_int, _vp, _c.c_size_t, _c.c_size_t, _c.POINTER(_vp)]),
     "sfmm_plan_device_bytes": (_c.c_size_t, [_vp]),
     "sfmm_plan_host_bytes": (_c.c_size_t, [_vp]),
     "sfmm_plan_bind_staged": (_c.c_int, [_vp, _vp, _c.c_size_t, _vp, _c.c_size_t, _vp]),
@@ -265,16 +266,21 @@ class Plan:
     With ``prepared=True`` the plan is only validated and grouped on the host
     (sfmm_plan_prepare); ``bind(dev_ptr, nbytes, stream)`` then copies its
     tables into caller device memory of ``device_bytes`` bytes
-    asynchronously (sfmm_plan_bind)."""
+    asynchronously (sfmm_plan_bind).  ``max_bytes`` is the most device
+    memory there will be for it (sfmm_plan_prepare_within)."""
 
-    def __init__(self, ctx, op, items, prepared=False):
+    def __init__(self, ctx, op, items, prepared=False, max_bytes=None):
         items = np.ascontiguousarray(items, dtype=ITEM_DTYPE)
         self.ctx = ctx
         self.op = op
         self.n = len(items)
         h = ctypes.c_void_p()
-        f = load().sfmm_plan_prepare if prepared else load().sfmm_plan_create
-        rc = f(ctx.handle, op, items.ctypes.data, len(items), ctypes.byref(h))
+        if prepared and max_bytes is not None:
+            rc = load().sfmm_plan_prepare_within(ctx.handle, op, items.ctypes.data, len(items), int(max_bytes),
+                                                 ctypes.byref(h))
+        else:
+            f = load().sfmm_plan_prepare if prepared else load().sfmm_plan_create
+            rc = f(ctx.handle, op, items.ctypes.data, len(items), ctypes.byref(h))
         _check(rc, ctx.handle, "sfmm_plan_prepare" if prepared else "sfmm_plan_create")
         self._h = h
 

@@ -150,6 +150,32 @@ constexpr uint32_t kMaxRounds = 4;
 
 size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
+// Device layout of a plan of repeated targets: items, targets, reduction
+// items, scratch blocks.
+size_t red_items_offset(size_t n_items, size_t n_targets)
+{
+    return align_up(align_up(n_items * sizeof(sfmm_item), 256) + n_targets * sizeof(sfmm::RedTarget), 256);
+}
+size_t scratch_offset(size_t n_items, size_t n_targets, size_t n_blocks)
+{
+    return align_up(red_items_offset(n_items, n_targets) + n_blocks * sizeof(sfmm::RedItem), 256);
+}
+
+// Items a run may span, of lane, team (or two octet) and octet kernels.
+constexpr size_t kRunLength[3] = {64, 16, 8};
+
+// The items of one launch, and their scratch blocks with runs of each length.
+struct Bucket {
+    size_t begin, end;
+    bool seg = false;  // runs share blocks
+    size_t blocks[3] = {}, reals[3] = {};
+};
+struct Layout {
+    int family;
+    bool team, pairs;
+    int run;  // index into kRunLength
+};
+
 // Reals a translation writes into its (scratch) target block.
 uint32_t written_reals(int op, const sfmm_item &it)
 {
@@ -216,9 +242,9 @@ private:
 // are applied in list order by rounds (the k-th item of a target runs in
 // launch round k); otherwise every item writes its own scratch block and a
 // segmented reduction adds a target's blocks in list order (reduce.hip).
-// `compact`: repeated targets run on the kernels of the longest runs the
-// family has, for the fewest scratch blocks.
-int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm_plan &plan, bool compact)
+// A plan that would need more than `max_bytes` of device memory takes kernels
+// of longer runs if those fit.
+int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm_plan &plan, size_t max_bytes)
 {
     if (op < SFMM_M2M || op > SFMM_L2L) return fail(ctx, SFMM_ERR_LOGIC, "solidfmm: unknown operator");
     if (n && !items) return fail(ctx, SFMM_ERR_LOGIC, "solidfmm: null item list");
@@ -327,48 +353,94 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
     }
     // FP64 lane and MFMA kernels in scratch mode share one scratch block
     // among the items of a run: consecutive items of a launch, within one
-    // 64-item wave (lane kernels) or group of 8 (octet kernels) or 16 (team
-    // kernels), with the same target and orders and a nonzero shift (the
-    // kernels add a run's results across lanes).  follows[k]: item k can join
-    // the run of item k - 1.
+    // 64-item wave (lane kernels) or the group of 8 (octet kernels) or 16
+    // (team kernels, octets two by two) that a wave or team takes, with the
+    // same target and orders and a nonzero shift (the kernels add a run's
+    // results across lanes).  follows[k]: item k can join the run of item
+    // k - 1.
     const bool runs = plan.scratch && ctx->precision == SFMM_FP64;
     auto zero = [](const sfmm_item &it) { return it.x == 0.0 && it.y == 0.0 && it.z == 0.0; };
     std::vector<uint8_t> follows(runs ? m : 0);
-    uint64_t run_off = 0;
+    std::vector<Bucket> buckets;
     for (size_t begin = 0, end; begin < m; begin = end) {
         const Key &first = keys[begin];
         for (end = begin + 1; end < m && keys[end].round == first.round && keys[end].family == first.family &&
                               keys[end].pb == first.pb;)
             ++end;
-        const size_t count = end - begin;
-        const bool seg = runs && (first.family == sfmm::kLaneKernels || first.family == sfmm::kMfmaKernels);
-        size_t lane_runs = 0;  // runs within 64 items
-        for (size_t k = begin; seg && k < end; ++k) {
-            if (k > begin) {
-                const sfmm_item &a = items[keys[k - 1].index], &b = items[keys[k].index];
-                follows[k] = a.dst == b.dst && a.p_in == b.p_in && a.p_out == b.p_out && !zero(a) && !zero(b);
+        Bucket b{begin, end};
+        b.seg = runs && (first.family == sfmm::kLaneKernels || first.family == sfmm::kMfmaKernels);
+        for (size_t k = begin; plan.scratch && k < end; ++k) {
+            const sfmm_item &it = items[keys[k].index];
+            if (b.seg && k > begin) {
+                const sfmm_item &prev = items[keys[k - 1].index];
+                follows[k] = prev.dst == it.dst && prev.p_in == it.p_in && prev.p_out == it.p_out && !zero(prev) &&
+                             !zero(it);
             }
-            lane_runs += !(follows[k] && (k - begin) % 64 != 0);
+            for (int w = 0; w < 3; ++w)
+                if (!b.seg || !follows[k] || (k - begin) % kRunLength[w] == 0) {
+                    b.blocks[w]++;
+                    b.reals[w] += size_t(it.p_out) * (it.p_out + 1);
+                }
         }
-        int family = first.family;
-        if (family == sfmm::kMfmaKernels && choices_free && !ctx->tune[op][first.pb] &&
-            (seg ? sfmm::lanes_for_runs(op, first.pb, count, lane_runs, m) : sfmm::lanes_ahead(op, first.pb, count, shared)))
-            family = sfmm::kLaneKernels;
-        const bool lanes = family == sfmm::kLaneKernels;
-        const bool team = family == sfmm::kGenericKernel
-                              ? first.pb != sfmm::kGenericRest
-                              : (compact && plan.scratch) || count <= sfmm::team_items(op, first.pb);
-        const size_t wave = lanes ? 64 : team ? 16 : 8;  // items a run may span
-        plan.launches.push_back(
-            {{family, family == sfmm::kGenericKernel ? 0u : first.pb, false, ctx->precision, !plan.scratch},
-             ordered.size(), count, first.round});
+        buckets.push_back(b);
+    }
+    // The kernels of a bucket, and which of kRunLength its runs have.  `small`:
+    // the layout of the fewest scratch blocks.
+    auto layout = [&](const Bucket &b, bool small) {
+        const Key &first = keys[b.begin];
+        const size_t count = b.end - b.begin;
+        Layout l{first.family, false, false, 0};
+        if (l.family == sfmm::kGenericKernel) {
+            l.team = first.pb != sfmm::kGenericRest;
+        } else if (ctx->precision == SFMM_FP64 && l.family == sfmm::kMfmaKernels) {
+            if (choices_free && !ctx->tune[op][first.pb] &&
+                (b.seg ? (small && first.pb <= sfmm::kLaneSmallPlan) ||
+                             sfmm::lanes_for_runs(op, first.pb, count, b.blocks[0], m)
+                       : sfmm::lanes_ahead(op, first.pb, count, shared))) {
+                l.family = sfmm::kLaneKernels;
+            } else {
+                l.pairs = b.seg && small && sfmm::octet_pairs(first.pb, count);
+                l.team = !l.pairs && ((b.seg && small) || count <= sfmm::team_items(op, first.pb));
+                l.run = l.team || l.pairs ? 1 : 2;
+            }
+        }
+        return l;
+    };
+    // Where the scratch blocks of the faster kernels are too many for the memory
+    // there is, and those of longer runs are not, the plan takes the latter:
+    // always at the size of the allocation-free entry point's array, so that
+    // it and a plan of its own memory run the same kernels.
+    bool small = false;
+    if (plan.scratch) {
+        auto bytes = [&](bool sm) {
+            size_t blocks = 0, reals = 0;
+            for (const Bucket &b : buckets) {
+                const int w = layout(b, sm).run;
+                blocks += b.blocks[w];
+                reals += b.reals[w];
+            }
+            return scratch_offset(m, seen.size(), blocks) + reals * sizeof(double);
+        };
+        const size_t need = bytes(false), least = bytes(true);
+        for (size_t limit : {size_t(SFMM_NOALLOC_SCRATCH_BYTES), max_bytes})
+            small = small || (need > limit && least <= limit);
+    }
+    uint64_t run_off = 0;
+    for (const Bucket &b : buckets) {
+        const Layout l = layout(b, small);
+        const bool generic = l.family == sfmm::kGenericKernel;
+        const uint32_t pb = keys[b.begin].pb;
+        plan.launches.push_back({{l.family, generic ? 0u : pb, false, ctx->precision, !plan.scratch},
+                                 ordered.size(), b.end - b.begin, keys[b.begin].round});
         sfmm::KernelChoice &choice = plan.launches.back().k;
-        choice.seg = seg;
-        choice.team = team;
-        choice.long_runs = seg && lanes && sfmm::long_runs(first.pb, count, lane_runs);
-        for (size_t k = begin; k < end; ++k) {
+        choice.seg = b.seg;
+        choice.team = l.team;
+        choice.pairs = l.pairs;
+        choice.long_runs = b.seg && l.family == sfmm::kLaneKernels &&
+                           sfmm::long_runs(pb, b.end - b.begin, b.blocks[0]);
+        for (size_t k = b.begin; k < b.end; ++k) {
             const Key &key = keys[k];
-            if (family == sfmm::kGenericKernel) {
+            if (generic) {
                 choice.pk = std::max({choice.pk, key.p_in, key.p_out});
             } else if (key.p_in != key.pb || key.p_out != key.pb) {
                 choice.rt = true;
@@ -376,14 +448,16 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
             sfmm_item it = items[key.index];
             if (plan.scratch) {
                 const uint32_t pos = list_pos[key.index];
-                if (!seg || !follows[k] || (k - begin) % wave == 0) {  // a block of its own in the scratch pool
-                    run_off = scratch_reals;
+                const size_t at = k - b.begin;
+                it.dst = run_off;
+                if (!b.seg || !follows[k] || at % kRunLength[l.run] == 0) {
+                    it.dst = run_off = scratch_reals;  // a block of its own in the scratch pool
                     scratch_reals += size_t(it.p_out) * (it.p_out + 1);
                 } else {
                     is_head[pos] = 0;
+                    if (l.pairs && at % 8 == 0) it.dst |= 1;  // octet.hpp, PAIRS
                 }
                 scr_off[pos] = run_off;
-                it.dst = run_off;
             }
             ordered.push_back(it);
         }
@@ -437,8 +511,8 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
     plan.n_targets = rt.size();
     // device layout and the host image of its first three parts
     plan.off_targets = align_up(m * sizeof(sfmm_item), 256);
-    plan.off_red_items = align_up(plan.off_targets + rt.size() * sizeof(sfmm::RedTarget), 256);
-    plan.off_scratch = align_up(plan.off_red_items + ri.size() * sizeof(sfmm::RedItem), 256);
+    plan.off_red_items = red_items_offset(m, rt.size());
+    plan.off_scratch = scratch_offset(m, rt.size(), ri.size());
     plan.dev_bytes = plan.scratch ? plan.off_scratch + scratch_reals * sizeof(double) : m * sizeof(sfmm_item);
     const size_t image = plan.scratch ? plan.off_scratch : m * sizeof(sfmm_item);
     plan.blob.assign(image, 0);
@@ -684,13 +758,14 @@ namespace {
 
 // Validation and grouping into a new plan with no device memory yet (its
 // device image stays on the host).
-int prepare_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm_plan **out, bool compact = false)
+int prepare_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm_plan **out,
+                 size_t max_bytes = ~size_t(0))
 {
     sfmm_plan *plan = new (std::nothrow) sfmm_plan;
     if (!plan) return fail(ctx, SFMM_ERR_ALLOC, "solidfmm: out of host memory");
     int rc;
     try {
-        rc = build_plan(ctx, op, items, n, *plan, compact);
+        rc = build_plan(ctx, op, items, n, *plan, max_bytes);
     } catch (const std::bad_alloc &) {
         rc = fail(ctx, SFMM_ERR_ALLOC, "solidfmm: out of host memory");
     }
@@ -739,6 +814,12 @@ int sfmm_plan_create(sfmm_context *ctx, int op, const sfmm_item *items, size_t n
 
 int sfmm_plan_prepare(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm_plan **out)
 {
+    return sfmm_plan_prepare_within(ctx, op, items, n, ~size_t(0), out);
+}
+
+int sfmm_plan_prepare_within(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, size_t max_bytes,
+                             sfmm_plan **out)
+{
     if (!ctx || !out) return SFMM_ERR_LOGIC;
     *out = nullptr;
     // build_plan reads only the context's order and kernel choices: copy
@@ -753,7 +834,7 @@ int sfmm_plan_prepare(sfmm_context *ctx, int op, const sfmm_item *items, size_t 
         std::memcpy(view.tune, ctx->tune, sizeof(view.tune));
     }
     sfmm_plan *plan = nullptr;
-    const int rc = prepare_plan(&view, op, items, n, &plan);
+    const int rc = prepare_plan(&view, op, items, n, &plan, max_bytes);
     if (rc != SFMM_OK) {
         std::lock_guard<std::mutex> lock(ctx->mu);
         ctx->err = view.err;
@@ -917,11 +998,6 @@ int sfmm_translate_noalloc(sfmm_context *ctx, int op, const sfmm_item *host_item
     int rc = sfmm_plan_prepare(ctx, op, host_items, n, &plan);  // host memory only
     if (rc != SFMM_OK) return rc;
     std::lock_guard<std::mutex> lock(ctx->mu);
-    if (plan->dev_bytes > kNoAllocBytes && plan->scratch) {
-        delete plan;
-        rc = prepare_plan(ctx, op, host_items, n, &plan, true);
-        if (rc != SFMM_OK) return rc;
-    }
     if (plan->dev_bytes > kNoAllocBytes) {
         rc = fail(ctx, SFMM_ERR_LOGIC,
                   "solidfmm: the list needs " + std::to_string(plan->dev_bytes) +

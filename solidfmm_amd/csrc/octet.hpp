@@ -266,9 +266,11 @@ constexpr int side_by_side(int pb) { return pb <= 8 || pb == 15 || pb == 16 ? 1 
 // >= p_out (L2L: >= min(p_in, p_out), translations.cpp:412) are not stored.
 // mode 1: target += T(source); 0: target block = T(source); 2: as 0, with
 // the items of a run (consecutive translations of the group with one block)
-// added across lanes and stored by the run's first.  `late` is called once
-// the registers of the triangle are free.
-template <int OP, int PB, class F>
+// added across lanes and stored by the run's first.  PAIRS: mode 2 with runs
+// that may go on from an even group into the odd one after it; bit 0 of such a
+// group's first block offset says that the block has the run's beginning
+// already.  `late` is called once the registers of the triangle are free.
+template <int OP, int PB, bool PAIRS, class F>
 __device__ __forceinline__ void translate_group(const double *__restrict__ src_pool, double *__restrict__ dst_pool,
                                                 const Group &G, uint32_t n_items, uint32_t g, const double *tab,
                                                 double *buf, int lane, int mode, F &&late)
@@ -293,8 +295,12 @@ __device__ __forceinline__ void translate_group(const double *__restrict__ src_p
     const int pout_w = wave_max5(active ? p_dst : 0u);
 
     const double *__restrict__ S = active ? src_pool + G.src + 2 * c : kZeroBlock;
-    double *__restrict__ D = dst_pool + G.dst + 2 * c;
-    const double *__restrict__ O = active && acc ? D : kZeroBlock;
+    const uint64_t block = PAIRS ? G.dst & ~uint64_t(1) : G.dst;
+    const bool joins = PAIRS && (G.dst & 1);
+    // the group before has stored to the CU's cache before this one loads
+    if (__ballot(joins)) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    double *__restrict__ D = dst_pool + block + 2 * c;
+    const double *__restrict__ O = active && (acc || joins) ? D : kZeroBlock;
 
     // pieces c + 8 i of degree n, zeros beyond the degree or the order
     auto fetch = [&](auto nc, const double *p, uint32_t order, auto &v) {
@@ -328,7 +334,7 @@ __device__ __forceinline__ void translate_group(const double *__restrict__ src_p
     uint32_t same = 0;
     bool store = active;
     if (mode == 2) {
-        const uint64_t key = active ? G.dst : ~uint64_t(tp);
+        const uint64_t key = active ? block : ~uint64_t(tp);
         const uint32_t lo32 = uint32_t(key), hi32 = uint32_t(key >> 32);
         static_for<0, 3>([&](auto jc) {
             constexpr int j = decltype(jc)::value;
@@ -553,7 +559,7 @@ __device__ __forceinline__ void translate_group(const double *__restrict__ src_p
         // target += source over the common degrees (translations.cpp:539-547,
         // 596-604)
         const double *s = src_pool + G.src;
-        double *d = dst_pool + G.dst;
+        double *d = dst_pool + block;
         const int len = int(p_end * (p_end + 1));
         for (int i = c; i < len; i += kItems) d[i] = (acc ? d[i] : 0.0) + s[i];
     }
@@ -569,7 +575,7 @@ constexpr size_t lds_bytes(int op, int pb)
 
 // Persistent workgroups: stage the swap operands in LDS, then each wave takes
 // groups of eight translations.
-template <int OP, int PB>
+template <int OP, int PB, bool PAIRS>
 __global__ void __launch_bounds__(64 * waves(PB)) __attribute__((amdgpu_waves_per_eu(per_simd(PB))))
     k_octet(const double *__restrict__ src_pool, double *__restrict__ dst_pool, const sfmm_item *__restrict__ items,
             uint32_t n_items, const double *__restrict__ tables_m, const double *__restrict__ tables_l, int mode)
@@ -578,7 +584,8 @@ __global__ void __launch_bounds__(64 * waves(PB)) __attribute__((amdgpu_waves_pe
     constexpr int W = waves(PB), SIZE = table_size(PB);
     const int lane = int(threadIdx.x & 63), wave = int(threadIdx.x >> 6);
     const uint32_t groups = (n_items + kItems - 1) / kItems;
-    uint32_t g = blockIdx.x * W + uint32_t(wave);
+    constexpr uint32_t kPair = PAIRS ? 1 : 0;  // a wave takes two groups in a row
+    uint32_t g = (blockIdx.x * W + uint32_t(wave)) << kPair;
     Group next{};
     if (g < groups) next.load(items, n_items, g, lane);
     const double2 *from_m = reinterpret_cast<const double2 *>(OP == SFMM_L2L ? tables_l : tables_m);
@@ -595,13 +602,13 @@ __global__ void __launch_bounds__(64 * waves(PB)) __attribute__((amdgpu_waves_pe
     while (g < groups) {
         const Group G = next;
         const uint32_t cur = g;
-        g += gridDim.x * W;
+        g += (cur & kPair) == kPair ? ((gridDim.x * W) << kPair) - kPair : 1;
         if (kEarly && g < groups) next.load(items, n_items, g, lane);
         // an opaque zero offset per group keeps the compiler from holding
         // operands in registers across groups
         int base = 0;
         asm volatile("" : "+s"(base));
-        translate_group<OP, PB>(src_pool, dst_pool, G, n_items, cur, lds + base, buf, lane, mode, [&] {
+        translate_group<OP, PB, PAIRS>(src_pool, dst_pool, G, n_items, cur, lds + base, buf, lane, mode, [&] {
             if (!kEarly && g < groups) next.load(items, n_items, g, lane);
         });
     }
@@ -609,24 +616,27 @@ __global__ void __launch_bounds__(64 * waves(PB)) __attribute__((amdgpu_waves_pe
 
 using fn_t = void (*)(const double *, double *, const sfmm_item *, uint32_t, const double *, const double *, int);
 
-template <int OP, int... Ps>
+template <int OP, bool PAIRS, int FIRST, int... Ps>
 constexpr auto make_table(std::integer_sequence<int, Ps...>)
 {
     struct T {
         fn_t f[sizeof...(Ps)];
-    } t{{&k_octet<OP, Ps + 1>...}};
+    } t{{&k_octet<OP, FIRST + Ps, PAIRS>...}};
     return t;
 }
 
 template <int OP>
 hipError_t launch_op(uint32_t pb, const sfmm_item *items, size_t n, const double *src, double *dst,
-                     hipStream_t stream, int mode)
+                     hipStream_t stream, int mode, bool pairs)
 {
-    static const auto t = make_table<OP>(std::make_integer_sequence<int, max_order(OP)>{});
+    static const auto single = make_table<OP, false, 1>(std::make_integer_sequence<int, max_order(OP)>{});
+    static const auto paired =
+        make_table<OP, true, kPairsMin>(std::make_integer_sequence<int, kPairsMax - kPairsMin + 1>{});
     if (pb < 1 || pb > uint32_t(max_order(OP))) return hipErrorInvalidValue;
+    if (pairs && (mode != 2 || pb < kPairsMin || pb > kPairsMax)) return hipErrorInvalidValue;
     const double *table = device_table();
     if (!table) return hipErrorOutOfMemory;
-    const fn_t f = t.f[pb - 1];
+    const fn_t f = pairs ? paired.f[pb - kPairsMin] : single.f[pb - 1];
     const size_t lds = lds_bytes(OP, int(pb));
     if (lds > 64 * 1024) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(f),
@@ -634,8 +644,8 @@ hipError_t launch_op(uint32_t pb, const sfmm_item *items, size_t n, const double
         if (e != hipSuccess) return e;
     }
     const size_t w = size_t(waves(int(pb))), groups = (n + kItems - 1) / kItems;
-    const uint32_t grid =
-        persistent_grid(reinterpret_cast<const void *>(f), int(64 * w), (groups + w - 1) / w, lds);
+    const size_t units = pairs ? (groups + 1) / 2 : groups;  // what a wave takes at a time
+    const uint32_t grid = persistent_grid(reinterpret_cast<const void *>(f), int(64 * w), (units + w - 1) / w, lds);
     hipLaunchKernelGGL(f, dim3(grid), dim3(uint32_t(64 * w)), uint32_t(lds), stream, src, dst, items, uint32_t(n),
                        table, table + table_size(kMaxOrder), mode);
     return hipGetLastError();

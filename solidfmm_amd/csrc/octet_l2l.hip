@@ -4,7 +4,8 @@
 namespace sfmm {
 namespace octet {
 
-template hipError_t launch_op<SFMM_L2L>(uint32_t, const sfmm_item *, size_t, const double *, double *, hipStream_t, int);
+template hipError_t launch_op<SFMM_L2L>(uint32_t, const sfmm_item *, size_t, const double *, double *, hipStream_t, int,
+                                           bool);
 
 }  // namespace octet
 }  // namespace sfmm

@@ -138,6 +138,7 @@ struct sfmm_server {
     void *arena_mem = nullptr;
     unsigned char *host_pool = nullptr;  // pinned: plan tables pass through it
     std::unique_ptr<Arena> arena, host_arena;
+    size_t plan_bytes = 0;  // most device memory a plan can get in the arena
     std::vector<int32_t> readers[2], writers[2];
     hipEvent_t ref = nullptr;
     std::chrono::steady_clock::time_point t0;
@@ -356,7 +357,7 @@ struct sfmm_server {
             to_prepare.pop_front();
             lock.unlock();
             sfmm_plan *plan = nullptr;
-            const int rc = sfmm_plan_prepare(ctx, r->op, r->items.data(), r->items.size(), &plan);
+            const int rc = sfmm_plan_prepare_within(ctx, r->op, r->items.data(), r->items.size(), plan_bytes, &plan);
             // stage the tables in pinned memory here, off the scheduler
             size_t off = 0, len = 0;
             bool staged = false;
@@ -435,6 +436,7 @@ int sfmm_server_create(sfmm_context *ctx, double *m_pool, size_t m_len, double *
         return e == hipErrorOutOfMemory ? SFMM_ERR_ALLOC : SFMM_ERR_HIP;
     }
     sv->t0 = std::chrono::steady_clock::now();
+    sv->plan_bytes = arena_bytes / kAlign * kAlign;
     sv->arena.reset(new Arena(arena_bytes));
     sv->host_arena.reset(new Arena(arena_bytes));
     sfmm_server *raw = sv.get();

@@ -245,9 +245,9 @@ hipError_t launch_kernel(int op, const KernelChoice &k, const sfmm_item *items, 
         const int mode = (!k.acc && k.seg) ? 2 : acc;
         if (k.team) return launch_team(op, k.pk, items, n, src, dst, stream, mode);
         switch (op) {
-        case SFMM_M2M: return octet::launch_op<SFMM_M2M>(k.pk, items, n, src, dst, stream, mode);
-        case SFMM_M2L: return octet::launch_op<SFMM_M2L>(k.pk, items, n, src, dst, stream, mode);
-        default: return octet::launch_op<SFMM_L2L>(k.pk, items, n, src, dst, stream, mode);
+        case SFMM_M2M: return octet::launch_op<SFMM_M2M>(k.pk, items, n, src, dst, stream, mode, k.pairs);
+        case SFMM_M2L: return octet::launch_op<SFMM_M2L>(k.pk, items, n, src, dst, stream, mode, k.pairs);
+        default: return octet::launch_op<SFMM_L2L>(k.pk, items, n, src, dst, stream, mode, k.pairs);
         }
     }
     default:

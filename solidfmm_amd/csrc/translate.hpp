@@ -94,7 +94,9 @@ namespace octet {
 constexpr int max_order(int op) { return op == SFMM_M2L ? 22 : 24; }
 template <int OP>
 hipError_t launch_op(uint32_t pb, const sfmm_item *items, size_t n, const double *src, double *dst,
-                     hipStream_t stream, int mode);
+                     hipStream_t stream, int mode, bool pairs);
+// Orders whose kernels have a variant with runs of up to two groups (`pairs`).
+inline constexpr uint32_t kPairsMin = 13, kPairsMax = 17;
 }  // namespace octet
 
 // Largest list of orders up to pb that the MFMA family sends to the team
@@ -106,6 +108,18 @@ size_t team_items(int op, uint32_t pb);
 // in lane waves.
 bool lanes_ahead(int op, uint32_t pb, size_t n, bool shared);
 bool lanes_for_runs(int op, uint32_t pb, size_t n, size_t runs, size_t total);
+
+// Kernels of the plans of the fewest scratch blocks: up to order 12 lanes, with
+// runs of 64, above it team kernels or octets in pairs, with runs of 16.  Pairs
+// take lists that fill the chip twice over where a team takes longer than the
+// former one-wave-per-16 kernel did: M2L of 300,000 items in runs of 24, that
+// kernel, team, pairs, octets (us): order 14 487, 552, 349, 326; 16 601, 597,
+// 434, 412; 18 992, 820, 720, 700.
+inline constexpr uint32_t kLaneSmallPlan = kLaneMax;
+constexpr bool octet_pairs(uint32_t pb, size_t n)
+{
+    return pb >= octet::kPairsMin && pb <= octet::kPairsMax && n > 32768;
+}
 
 // Launch bucket of an FP64 item of the generic family, by its larger order:
 // 32 (orders 25 to 32) and kTeamMax (33 to 48) run on team kernels of their
@@ -135,6 +149,8 @@ struct KernelChoice {
     // MFMA and generic families: the team kernels, not the octet and generic
     // ones.  Decided with the runs, which are as long as the kernel's groups.
     bool team = false;
+    // octet kernels: the variant with runs of up to two groups
+    bool pairs = false;
 };
 
 // Segmented reduction: target block t += sum of its items' scratch blocks,

@@ -16,7 +16,7 @@ of HIP streams ("slots"):
   queue), so every cell sees its updates in arrival order and the pools end
   exactly as if the requests had run one by one.
 * Preparation.  On arrival a request's plan is validated and grouped on
-  the host by a pool of worker threads (sfmm_plan_prepare; the C call
+  the host by a pool of worker threads (sfmm_plan_prepare_within; the C call
   releases the interpreter lock), while the GPU runs earlier requests.
 * Execution.  On admission the prepared tables are copied into the arena
   and the kernels launched on the slot's stream (sfmm_plan_bind: no device
@@ -167,7 +167,8 @@ class Server:
         max_inflight = 0
         blocked = {"prepare": 0, "slot": 0, "arena": 0, "hazard": 0}
         pool = ThreadPoolExecutor(max_workers=self.workers)
-        prepare = lambda r: self._Plan(self.ctx, r.op, r.items, prepared=True)  # noqa: E731
+        most = self.arena.size // ALIGN * ALIGN
+        prepare = lambda r: self._Plan(self.ctx, r.op, r.items, prepared=True, max_bytes=most)  # noqa: E731
         while pending or waiting or inflight:
             now = time.perf_counter() - t0
             while pending and (not realtime or pending[0].arrival <= now):
