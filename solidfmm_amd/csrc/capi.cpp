@@ -257,6 +257,8 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
     std::vector<Key> keys;
     keys.reserve(n);
     FlatMap seen;  // target -> occurrences so far
+    uint32_t *occurred = nullptr;  // those of last_dst: neighbours often share a target
+    uint64_t last_dst = 0;
     size_t src_begin = ~size_t(0), src_read = 0;  // first source, reals read
     uint32_t rounds = 0;
     // kernel family per (p_in, p_out), filled on first use: lists repeat a
@@ -287,7 +289,9 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
         const uint32_t pb = std::max(it.p_in, it.p_out);
         const int fam = small_m2l && pb >= 9 && pb <= 11 && !ctx->tune[op][pb] ? sfmm::kLaneKernels : fc;
         bool fresh;
-        const uint32_t round = seen.get(it.dst, 0, fresh)++;
+        if (!occurred || it.dst != last_dst) occurred = &seen.get(it.dst, 0, fresh);
+        last_dst = it.dst;
+        const uint32_t round = (*occurred)++;
         rounds = std::max(rounds, round + 1);
         const size_t src_end = it.src + size_t(it.p_in) * (it.p_in + 1);
         plan.src_extent = std::max(plan.src_extent, src_end);
@@ -472,11 +476,12 @@ int build_plan(sfmm_context *ctx, int op, const sfmm_item *items, size_t n, sfmm
         std::vector<uint32_t> count;
         std::vector<uint32_t> of_pos(m);  // target id per list position
         size_t pos = 0, heads = 0;
+        uint32_t t = 0;
         for (size_t i = 0; i < n; ++i) {
             const sfmm_item &it = items[i];
             if (it.p_in == 0 || it.p_out == 0) continue;
-            bool fresh;
-            const uint32_t t = tid.get(it.dst, uint32_t(rt.size()), fresh);
+            bool fresh = false;
+            if (rt.empty() || it.dst != rt[t].dst) t = tid.get(it.dst, uint32_t(rt.size()), fresh);
             if (fresh) {
                 rt.push_back({it.dst, 0, 0, 0, 0});
                 count.push_back(0);
