@@ -99,12 +99,89 @@ struct cplx {
 };
 __device__ __forceinline__ cplx mul(cplx a, cplx b) { return {a.c * b.c - a.s * b.s, a.s * b.c + a.c * b.s}; }
 
+// Values in twice the precision (hi + lo).  A power of a rounded value is off
+// by its error times the exponent, and by as much again where it comes from
+// squarings: with angles in 64 bits, M2L of order 25 had a median error of
+// 1.08e-14 a degree, 28 of 1.72e-14, where the one-workgroup kernel, which
+// multiplies up, has 9.2e-15 and 1.42e-14; with these 8.7e-15 and 1.24e-14.
+struct Wide {
+    double hi, lo;
+};
+__device__ __forceinline__ Wide normal(double hi, double lo)
+{
+    const double h = hi + lo;
+    return {h, lo - (h - hi)};
+}
+__device__ __forceinline__ Wide two_sum(double a, double b)
+{
+    const double s = a + b, bb = s - a;
+    return {s, (a - (s - bb)) + (b - bb)};
+}
+__device__ __forceinline__ Wide two_prod(double a, double b)
+{
+    const double p = a * b;
+    return {p, __builtin_fma(a, b, -p)};
+}
+__device__ __forceinline__ Wide mul(Wide a, Wide b)
+{
+    const Wide p = two_prod(a.hi, b.hi);
+    return normal(p.hi, __builtin_fma(a.hi, b.lo, __builtin_fma(a.lo, b.hi, p.lo)));
+}
+
+// |(x, y, z)| and its inverse.
+struct Distance {
+    Wide r, inv;
+};
+__device__ __forceinline__ Distance distance(double x, double y, double z)
+{
+    const Wide xx = two_prod(x, x), yy = two_prod(y, y), zz = two_prod(z, z);
+    const Wide s = two_sum(xx.hi, yy.hi), t = two_sum(s.hi, zz.hi);
+    const double lo = t.lo + s.lo + (xx.lo + yy.lo + zz.lo);  // r^2 = t.hi + lo
+    const double inv = 1.0 / sqrt(t.hi);
+    Wide r = two_prod(t.hi, inv);
+    r.lo += lo * inv;
+    const Wide v = two_prod(r.hi, inv);
+    const double e = (1.0 - v.hi) - v.lo - r.lo * inv;  // 1 - r^2 inv^2
+    return {normal(r.hi, r.lo + 0.5 * e * r.hi), normal(inv, 0.5 * e * inv)};
+}
+
+// e^{i theta}, squared and once more.
+struct Turn {
+    Wide c, s;
+};
+__device__ __forceinline__ Turn square(const Turn &a)
+{
+    const Wide cc = two_prod(a.c.hi, a.c.hi), ss = two_prod(a.s.hi, a.s.hi), cs = two_prod(a.c.hi, a.s.hi);
+    const Wide d = two_sum(cc.hi, -ss.hi);
+    const double dl = d.lo + (cc.lo - ss.lo) + 2.0 * (a.c.hi * a.c.lo - a.s.hi * a.s.lo);
+    const double sl = cs.lo + a.c.hi * a.s.lo + a.s.hi * a.c.lo;
+    return {normal(d.hi, dl), normal(2.0 * cs.hi, 2.0 * sl)};
+}
+__device__ __forceinline__ cplx rounded(const Turn &a) { return {a.c.hi, a.s.hi}; }
+
+// Kernels of this many chunks or more have Wide angles: orders above 24, at 1
+// to 4 % of their time (M2L of order 32, 2,003 items 37.4 -> 37.8 us).  Up to 24
+// the errors are those of the kernels before, and short lists would take 8 %
+// longer.
+inline constexpr int kWide = 4;
+
 // e^{i m theta} for m = 2 (q + 4 j) + e: squares for e^{2i}, e^{4i}, e^{8i},
 // then one product per slot.
 template <int NJX>
-__device__ __forceinline__ void powers(cplx one, int q, double (&c)[2][NJX], double (&s)[2][NJX])
+__device__ __forceinline__ void powers(const Turn &t1, int q, double (&c)[2][NJX], double (&s)[2][NJX])
 {
-    const cplx two = mul(one, one), four = mul(two, two), eight = mul(four, four);
+    const cplx one = rounded(t1);
+    cplx two, four, eight;
+    if constexpr (NJX >= kWide) {
+        const Turn t2 = square(t1), t4 = square(t2);
+        two = rounded(t2);
+        four = rounded(t4);
+        eight = rounded(square(t4));
+    } else {
+        two = mul(one, one);
+        four = mul(two, two);
+        eight = mul(four, four);
+    }
     cplx p{1.0, 0.0};
     if (q & 1) p = two;
     if (q & 2) p = (q & 1) ? mul(two, four) : four;
@@ -372,15 +449,21 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     const double rho2 = x * x + y * y;
     const double rho = sqrt(rho2);
     const double r = sqrt(rho2 + z * z);
-    const double rinv = 1.0 / r;
-    cplx ea{1.0, 0.0};
-    if (rho != 0.0) {
+    const double rinv = 1.0 / r;  // of the rounded r: M2M and L2L multiply by powers of both
+    Turn ea{{1.0, 0.0}, {0.0, 0.0}}, eb{{z * rinv, 0.0}, {-rho * rinv, 0.0}};
+    if constexpr (NJX >= kWide) {
+        const Distance xyz = distance(x, y, z), xy = distance(x, y, 0.0);
+        eb.c = mul({z, 0.0}, xyz.inv);
+        if (rho != 0.0) {
+            ea = {mul({y, 0.0}, xy.inv), mul({x, 0.0}, xy.inv)};
+            eb.s = mul({-xy.r.hi, -xy.r.lo}, xyz.inv);
+        }
+    } else if (rho != 0.0) {
         const double qq = 1.0 / rho;
-        ea = cplx{y * qq, x * qq};
+        ea = {{y * qq, 0.0}, {x * qq, 0.0}};
     }
     constexpr bool kInLds = NJX >= kRotLds;
     double ca[2][NJX], sa[2][NJX], cb[2][NJX], sb[2][NJX];
-    const cplx eb{z * rinv, -rho * rinv};
     if constexpr (kInLds) {
         if (wave < 2) {
             powers<NJX>(wave ? eb : ea, q, ca, sa);
@@ -534,6 +617,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
         };
         if constexpr (NJX <= kSmall) {
             const int chunks = (max(nk, nn) + 3) / 4;
+            bool slow = false;
             static_for<1, 2 * NJX + 1>([&](auto ncc) {
                 constexpr int NC = decltype(ncc)::value;
                 if (chunks == NC) {
@@ -562,10 +646,14 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
                             }
                         });
                     });
-                    if (unbounded(br, bi)) return one_sided();
-                    static_for<0, NC>([&](auto oc) { put(4 * decltype(oc)::value + q, dr[decltype(oc)::value], di[decltype(oc)::value]); });
+                    if constexpr (OP != SFMM_M2L) slow = unbounded(br, bi);
+                    if (!slow)
+                        static_for<0, NC>([&](auto oc) { put(4 * decltype(oc)::value + q, dr[decltype(oc)::value], di[decltype(oc)::value]); });
                 }
             });
+            if constexpr (OP != SFMM_M2L) {
+                if (slow) one_sided();
+            }
         } else {
             double br[2 * NJX], bi[2 * NJX];
             static_for<0, 2 * NJX>([&](auto cc) {
