@@ -640,6 +640,18 @@ __global__ void __launch_bounds__(64)
     l2p_run<D>(pts, pool, phi, grad, cr, R, H, at);
 }
 
+// Calls launch(first cell, cells, workgroups) for n_cells cells, `run` a
+// workgroup of 64 threads, in launches of fewer than 2^32 threads.
+template <class F>
+void launch_runs(size_t n_cells, uint32_t run, F &&launch)
+{
+    const size_t most = (size_t(1) << 24) * run;
+    for (size_t first = 0; first < n_cells; first += most) {
+        const size_t n = std::min(n_cells - first, most);
+        launch(first, uint32_t(n), uint32_t((n + run - 1) / run));
+    }
+}
+
 // Cells per wave: about `waves` waves, which is where P2M and L2P measured
 // best (one long round of L2P's resident waves, three shorter ones of P2M's).
 uint32_t run_length(size_t n_cells, size_t waves)
@@ -664,8 +676,9 @@ hipError_t p2m_d(const double *pts, const sfmm_cell *cells, size_t n_cells, uint
     const size_t block = size_t(staged_rows(int(max_order))) * D * sizeof(double);
     const size_t fit = std::max(block ? kStageBytes / block : kRun, size_t(1));
     const uint32_t run = std::min(run_length(n_cells, kWavesP2M), uint32_t(fit));
-    hipLaunchKernelGGL(k_p2m<D>, dim3(uint32_t((n_cells + run - 1) / run)), dim3(64), run * block, stream, pts, cells,
-                       uint32_t(n_cells), pool, run);
+    launch_runs(n_cells, run, [&](size_t first, uint32_t n, uint32_t groups) {
+        hipLaunchKernelGGL(k_p2m<D>, dim3(groups), dim3(64), run * block, stream, pts, cells + first, n, pool, run);
+    });
     return hipGetLastError();
 }
 
@@ -681,8 +694,10 @@ hipError_t l2p_d(const double *pts, const sfmm_cell *cells, size_t n_cells, uint
     }
     const uint32_t run = run_length(n_cells, kWavesL2P);
     const uint32_t split = n_cells < 2048 ? 4 : 1;  // few cells: their chunks side by side
-    hipLaunchKernelGGL(k_l2p<D>, dim3(uint32_t((n_cells + run - 1) / run), split), dim3(64), 0, stream, pts, cells,
-                       uint32_t(n_cells), pool, phi, grad, run);
+    launch_runs(n_cells, run, [&](size_t first, uint32_t n, uint32_t groups) {
+        hipLaunchKernelGGL(k_l2p<D>, dim3(groups, split), dim3(64), 0, stream, pts, cells + first, n, pool, phi, grad,
+                           run);
+    });
     return hipGetLastError();
 }
 

@@ -1,6 +1,7 @@
 // Launches of the team kernels (team.hpp).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 
 #include "../../include/solidfmm_gpu.h"
@@ -67,8 +68,13 @@ hipError_t launch_team(int op, uint32_t pc, const sfmm_item *items, size_t n, co
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, int(kLds));
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL(f, dim3(uint32_t(groups)), dim3(64 * waves), lds, stream, src, dst, items, uint32_t(n), table,
-                       fac, int(pc), tl, mode);
+    // a launch holds fewer than 2^32 threads
+    constexpr size_t kMost = size_t(1) << 22;
+    for (size_t g = 0; g < groups; g += kMost) {
+        const size_t first = g << tl;
+        hipLaunchKernelGGL(f, dim3(uint32_t(std::min(groups - g, kMost))), dim3(64 * waves), lds, stream, src, dst,
+                           items + first, uint32_t(n - first), table, fac, int(pc), tl, mode);
+    }
     return hipGetLastError();
 }
 
