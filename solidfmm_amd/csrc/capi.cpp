@@ -1478,8 +1478,8 @@ int sfmm_translate_host(sfmm_context *ctx, int op, const sfmm_item *items, size_
 struct sfmm_cellset {
     sfmm_context *ctx = nullptr;
     sfmm_cell *d_cells = nullptr;
-    size_t n_cells = 0, n_points = 0, pool_extent = 0;
-    uint32_t max_order = 0;
+    size_t n_points = 0, pool_extent = 0;
+    sfmm::CellCounts counts;
     int dim = 1;
 };
 
@@ -1490,7 +1490,7 @@ int sfmm_cellset_create(sfmm_context *ctx, const sfmm_cell *cells, size_t n, siz
     *out = nullptr;
     if (n && !cells) return fail(ctx, SFMM_ERR_LOGIC, "solidfmm: null cell list");
     size_t extent = 0;
-    uint32_t max_order = 0;
+    sfmm::CellCounts counts;
     const uint32_t dim = n ? std::max(cells[0].dim, 1u) : 1u;
     if (dim > uint32_t(sfmm::kMaxParticleDim))
         return fail(ctx, SFMM_ERR_LOGIC, "solidfmm: particle expansions of dimension 1..4 only");
@@ -1501,15 +1501,14 @@ int sfmm_cellset_create(sfmm_context *ctx, const sfmm_cell *cells, size_t n, siz
         if (uint64_t(c.first) + c.count > n_points) return fail(ctx, SFMM_ERR_LOGIC, "solidfmm: cell points out of range");
         if (std::max(c.dim, 1u) != dim) return fail(ctx, SFMM_ERR_LOGIC, "solidfmm: cells of one set must share dim");
         extent = std::max<size_t>(extent, c.offset + size_t(dim) * c.order * (c.order + 1));
-        max_order = std::max(max_order, c.order);
+        counts.add(c);
     }
     sfmm_cellset *set = new (std::nothrow) sfmm_cellset;
     if (!set) return fail(ctx, SFMM_ERR_ALLOC, "solidfmm: out of host memory");
     set->ctx = ctx;
-    set->n_cells = n;
     set->n_points = n_points;
     set->pool_extent = extent;
-    set->max_order = max_order;
+    set->counts = counts;
     set->dim = int(dim);
     hipError_t e = hipSetDevice(ctx->device);
     if (e == hipSuccess && n) {
@@ -1539,11 +1538,10 @@ int sfmm_p2m(sfmm_cellset *set, const double *points, size_t n_points, double *p
     std::lock_guard<std::mutex> lock(ctx->mu);
     if (n_points < set->n_points || pool_len < set->pool_extent)
         return fail(ctx, SFMM_ERR_LOGIC, "solidfmm: points or pool shorter than the cell set needs");
-    if (set->n_cells && (!points || !pool)) return fail(ctx, SFMM_ERR_LOGIC, "solidfmm: null pointer");
+    if (set->counts.cells && (!points || !pool)) return fail(ctx, SFMM_ERR_LOGIC, "solidfmm: null pointer");
     hipError_t e = hipSetDevice(ctx->device);
     if (e == hipSuccess)
-        e = sfmm::launch_p2m(points, set->d_cells, set->n_cells, set->max_order, pool, set->dim,
-                             static_cast<hipStream_t>(stream));
+        e = sfmm::launch_p2m(points, set->d_cells, set->counts, pool, set->dim, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(ctx, e, "p2m launch");
     return SFMM_OK;
 }
@@ -1556,10 +1554,10 @@ int sfmm_l2p(sfmm_cellset *set, const double *points, size_t n_points, const dou
     std::lock_guard<std::mutex> lock(ctx->mu);
     if (n_points < set->n_points || pool_len < set->pool_extent)
         return fail(ctx, SFMM_ERR_LOGIC, "solidfmm: points or pool shorter than the cell set needs");
-    if (set->n_cells && (!points || !pool || !phi)) return fail(ctx, SFMM_ERR_LOGIC, "solidfmm: null pointer");
+    if (set->counts.cells && (!points || !pool || !phi)) return fail(ctx, SFMM_ERR_LOGIC, "solidfmm: null pointer");
     hipError_t e = hipSetDevice(ctx->device);
     if (e == hipSuccess)
-        e = sfmm::launch_l2p(points, set->d_cells, set->n_cells, set->max_order, pool, phi, grad, set->dim,
+        e = sfmm::launch_l2p(points, set->d_cells, set->counts, pool, phi, grad, set->dim,
                              static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(ctx, e, "l2p launch");
     return SFMM_OK;

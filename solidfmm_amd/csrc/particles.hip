@@ -27,16 +27,19 @@
 //          (d/dx -+ i d/dy) R_n^m = +-R_{n-1}^{m-+1},
 //        so the gradient needs no recurrence of its own.  The instruction's
 //        four blocks are four quads, each with the H of its own cell.
-// What bounds them: the FP64 pipe and the latency of a wave's chunk (about
-// four waves per SIMD are in flight).  One lane per coefficient with its own
-// O(n) recurrence per point (P2M) and one cell per wave with the gradient's
-// recurrences (L2P) took 2 to 12 times (P2M) and up to 2.5 times
-// (L2P) as long: P2M of 250,000 points, order 8, three charges, 24 points a
-// cell 157 -> 42 us (the multiplications would take 4 us, the bytes 10), L2P
-// of 500,000 points, order 10, 32 a cell 115 -> 77 us (11 and 12 us).
+// What bounds them: the FP64 pipe and the latency of a wave's chunk (the
+// registers leave three waves per SIMD, two of L2P with more than one charge).
+// The kernels per cell (one lane per coefficient with its own O(n) recurrence
+// per point, P2M; one lane per point with the gradient's recurrences, L2P) take
+// longer where a cell's points are no match for their lanes: P2M of 250,000
+// points, order 8, three charges, 24 a cell 157 and 42 us (the multiplications
+// would take 4 us, the bytes 10), L2P of 500,000 points, order 10, 32 a cell
+// on average 115 and 75 us (11 and 12 us).  They stay for the sets that
+// per_cell_p2m and per_cell_l2p name.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 
 #include "../../include/solidfmm_gpu.h"
@@ -652,8 +655,10 @@ void launch_runs(size_t n_cells, uint32_t run, F &&launch)
     }
 }
 
-// Cells per wave: about `waves` waves, which is where P2M and L2P measured
-// best (one long round of L2P's resident waves, three shorter ones of P2M's).
+// Cells per wave: about `waves` waves.  Over orders 4 to 16, 8 to 128 points a
+// cell and 2,000 to 500,000 points, half as many take 0.61 to 1.25 of P2M's
+// time (the least where 4,000 cells go two to a wave) and 0.85 to 1.38 of
+// L2P's, twice as many 0.90 to 1.15 and 0.83 to 1.45.
 uint32_t run_length(size_t n_cells, size_t waves)
 {
     const size_t r = (n_cells + waves - 1) / waves;
@@ -664,37 +669,95 @@ constexpr size_t kWavesP2M = 5632, kWavesL2P = 1792;
 // LDS (bytes) of P2M's staged blocks that leaves room for eight waves a CU.
 constexpr size_t kStageBytes = 9 * 1024;
 
-template <int D>
-hipError_t p2m_d(const double *pts, const sfmm_cell *cells, size_t n_cells, uint32_t max_order, double *pool,
-                 hipStream_t stream)
+// P2M takes a wave per cell where the cells have so few points that the walk
+// would mostly be for lanes without one: up to `few` points a cell (four times
+// that in the largest, a wave of its own in both kernels).  Where the kernel
+// per cell was no slower, in us against the walk's:
+//   orders to 10, a cell's coefficients one pass of a wave: up to 6 while the
+//   cells are in flight at once (30,000 points of order 8, one charge: 17 and
+//   22 at 4 a cell, 21 and 14 at 12), 4 of very few cells; of many cells 2 or
+//   3 from order 8 on, below it 1 and only up to two charges, since one
+//   more charge costs the walk less;
+//   above: 2 of few cells; of many 3 or 4, with one charge 1 and from order 20
+//   on 2 to 4, as the staged blocks leave the walk fewer waves (200,000 points
+//   of order 24, one charge: 1126 and 1634 at 3 a cell, 997 and 821 at 6).
+bool per_cell_p2m(const CellCounts &c, int dim)
 {
-    if (max_order > kWalkMax) {
-        const uint32_t grid = persistent_grid(reinterpret_cast<const void *>(&k_p2m_cell<D>), 64, n_cells);
-        hipLaunchKernelGGL(k_p2m_cell<D>, dim3(grid), dim3(64), 0, stream, pts, cells, uint32_t(n_cells), pool);
+    const uint32_t P = c.max_order;
+    size_t few;
+    if (P <= 10) {
+        if (c.cells <= 512) few = 4;
+        else if (c.cells <= 32768) few = 6;
+        else if (P >= 8) few = dim >= 3 && P > 8 ? 3 : 2;
+        else few = dim <= 2 ? 1 : 0;
+    } else if (c.cells < 1024) few = 2;
+    else if (dim == 1) few = P >= 24 ? 4 : P >= 20 ? 2 : 1;
+    else few = P >= 16 || dim == 4 ? 4 : 3;
+    return c.points <= few * c.cells && c.most <= 4 * few;
+}
+
+// L2P takes a wave per cell where cells fill their own chunks of 64 lanes so
+// well that the walk, whose runs share chunks, has few less to go through: one
+// of its chunks costs as much as 1 / (share + slope (P - 4)) of the kernel
+// per cell.  The cells must fill the chip as well, from `cells` times the
+// order on for cells of one chunk.  The lines are fitted to the times of both
+// kernels at orders 4 to 32, 1 to 1,000 points a cell and 2,000 to 1,000,000
+// points, where the chosen one is on average 0.4 % behind the faster.
+// 1,000,000 points of order 8, three charges, per cell and on the walk: 131
+// and 210 us at 64 points a cell, 311 and 164 at 24; of order 10, one charge,
+// 123 and 97 at 64.  Order 4 with all chunks in flight at once gains nothing
+// from the exchange through LDS with more than one charge (30,000 points, three
+// charges, 24 a cell: 8.8 and 10.9; 60,000 points, one charge, 12 a cell: 10.0
+// and 9.0).
+bool per_cell_l2p(const CellCounts &c, int dim)
+{
+    struct Line {
+        double share, slope;
+        uint32_t cells;
+    };
+    constexpr Line kLine[kMaxParticleDim] = {{0.40, 0.15, 375}, {0.45, 0.06, 256}, {0.35, 0.08, 192}, {0.40, 0.03, 128}};
+    const Line &line = kLine[dim - 1];
+    const uint32_t P = c.max_order;
+    if (P <= 4 && dim > 1 && c.most <= 64 && c.cells <= 5120) return true;
+    const size_t run = run_length(c.cells, kWavesL2P), runs = (c.cells + run - 1) / run;
+    const double walk = double(runs) * std::ceil(double(c.quads) * double(run) / double(16 * c.cells));
+    const uint64_t deepest = c.most / 64 + (c.most % 64 != 0);
+    return walk >= (line.share + line.slope * (int(P) - 4)) * double(c.chunks) &&
+           c.chunks >= deepest * line.cells * P;
+}
+
+template <int D>
+hipError_t p2m_d(const double *pts, const sfmm_cell *cells, const CellCounts &c, double *pool, hipStream_t stream)
+{
+    if (c.max_order > kWalkMax || per_cell_p2m(c, D)) {
+        const uint32_t grid = persistent_grid(reinterpret_cast<const void *>(&k_p2m_cell<D>), 64, c.cells);
+        hipLaunchKernelGGL(k_p2m_cell<D>, dim3(grid), dim3(64), 0, stream, pts, cells, uint32_t(c.cells), pool);
         return hipGetLastError();
     }
-    const size_t block = size_t(staged_rows(int(max_order))) * D * sizeof(double);
+    const size_t block = size_t(staged_rows(int(c.max_order))) * D * sizeof(double);
     const size_t fit = std::max(block ? kStageBytes / block : kRun, size_t(1));
-    const uint32_t run = std::min(run_length(n_cells, kWavesP2M), uint32_t(fit));
-    launch_runs(n_cells, run, [&](size_t first, uint32_t n, uint32_t groups) {
+    const uint32_t run = std::min(run_length(c.cells, kWavesP2M), uint32_t(fit));
+    launch_runs(c.cells, run, [&](size_t first, uint32_t n, uint32_t groups) {
         hipLaunchKernelGGL(k_p2m<D>, dim3(groups), dim3(64), run * block, stream, pts, cells + first, n, pool, run);
     });
     return hipGetLastError();
 }
 
 template <int D>
-hipError_t l2p_d(const double *pts, const sfmm_cell *cells, size_t n_cells, uint32_t max_order, const double *pool,
-                 double *phi, double *grad, hipStream_t stream)
+hipError_t l2p_d(const double *pts, const sfmm_cell *cells, const CellCounts &c, const double *pool, double *phi,
+                 double *grad, hipStream_t stream)
 {
-    if (max_order < kWalkMinL2P || max_order > kWalkMax) {
-        const uint32_t grid = persistent_grid(reinterpret_cast<const void *>(&k_l2p_cell<D>), 64, n_cells);
-        hipLaunchKernelGGL(k_l2p_cell<D>, dim3(grid), dim3(64), 0, stream, pts, cells, uint32_t(n_cells), pool, phi,
+    if (c.max_order < kWalkMinL2P || c.max_order > kWalkMax || per_cell_l2p(c, D)) {
+        const uint32_t grid = persistent_grid(reinterpret_cast<const void *>(&k_l2p_cell<D>), 64, c.cells);
+        hipLaunchKernelGGL(k_l2p_cell<D>, dim3(grid), dim3(64), 0, stream, pts, cells, uint32_t(c.cells), pool, phi,
                            grad);
         return hipGetLastError();
     }
-    const uint32_t run = run_length(n_cells, kWavesL2P);
-    const uint32_t split = n_cells < 2048 ? 4 : 1;  // few cells: their chunks side by side
-    launch_runs(n_cells, run, [&](size_t first, uint32_t n, uint32_t groups) {
+    const uint32_t run = run_length(c.cells, kWavesL2P);
+    // few cells: a run's chunks side by side, 30,000 points of order 10, 128 a
+    // cell, 10.9 us, one after the other 28.9
+    const uint32_t split = c.cells < 2048 ? 4 : 1;
+    launch_runs(c.cells, run, [&](size_t first, uint32_t n, uint32_t groups) {
         hipLaunchKernelGGL(k_l2p<D>, dim3(groups, split), dim3(64), 0, stream, pts, cells + first, n, pool, phi, grad,
                            run);
     });
@@ -703,30 +766,30 @@ hipError_t l2p_d(const double *pts, const sfmm_cell *cells, size_t n_cells, uint
 
 }  // namespace
 
-hipError_t launch_p2m(const double *pts, const sfmm_cell *cells, size_t n_cells, uint32_t max_order, double *pool,
-                      int dim, hipStream_t stream)
+hipError_t launch_p2m(const double *pts, const sfmm_cell *cells, const CellCounts &counts, double *pool, int dim,
+                      hipStream_t stream)
 {
-    if (n_cells == 0) return hipSuccess;
-    if (n_cells > 0xFFFFFFFFull) return hipErrorInvalidValue;
+    if (counts.cells == 0) return hipSuccess;
+    if (counts.cells > 0xFFFFFFFFull) return hipErrorInvalidValue;
     switch (dim) {
-    case 1: return p2m_d<1>(pts, cells, n_cells, max_order, pool, stream);
-    case 2: return p2m_d<2>(pts, cells, n_cells, max_order, pool, stream);
-    case 3: return p2m_d<3>(pts, cells, n_cells, max_order, pool, stream);
-    case 4: return p2m_d<4>(pts, cells, n_cells, max_order, pool, stream);
+    case 1: return p2m_d<1>(pts, cells, counts, pool, stream);
+    case 2: return p2m_d<2>(pts, cells, counts, pool, stream);
+    case 3: return p2m_d<3>(pts, cells, counts, pool, stream);
+    case 4: return p2m_d<4>(pts, cells, counts, pool, stream);
     default: return hipErrorInvalidValue;
     }
 }
 
-hipError_t launch_l2p(const double *pts, const sfmm_cell *cells, size_t n_cells, uint32_t max_order,
-                      const double *pool, double *phi, double *grad, int dim, hipStream_t stream)
+hipError_t launch_l2p(const double *pts, const sfmm_cell *cells, const CellCounts &counts, const double *pool,
+                      double *phi, double *grad, int dim, hipStream_t stream)
 {
-    if (n_cells == 0) return hipSuccess;
-    if (n_cells > 0xFFFFFFFFull) return hipErrorInvalidValue;
+    if (counts.cells == 0) return hipSuccess;
+    if (counts.cells > 0xFFFFFFFFull) return hipErrorInvalidValue;
     switch (dim) {
-    case 1: return l2p_d<1>(pts, cells, n_cells, max_order, pool, phi, grad, stream);
-    case 2: return l2p_d<2>(pts, cells, n_cells, max_order, pool, phi, grad, stream);
-    case 3: return l2p_d<3>(pts, cells, n_cells, max_order, pool, phi, grad, stream);
-    case 4: return l2p_d<4>(pts, cells, n_cells, max_order, pool, phi, grad, stream);
+    case 1: return l2p_d<1>(pts, cells, counts, pool, phi, grad, stream);
+    case 2: return l2p_d<2>(pts, cells, counts, pool, phi, grad, stream);
+    case 3: return l2p_d<3>(pts, cells, counts, pool, phi, grad, stream);
+    case 4: return l2p_d<4>(pts, cells, counts, pool, phi, grad, stream);
     default: return hipErrorInvalidValue;
     }
 }
