@@ -62,7 +62,8 @@ enum {
     SFMM_KERNELS_AUTO = 0, /* per order bucket: the autotuned family, else the default */
     SFMM_KERNELS_LANE = 1, /* one lane per translation, FP64 VALU (orders <= 12) */
     SFMM_KERNELS_MFMA = 2, /* 8 or 16 translations per group, swaps on MFMA (orders <= 24; FP32 contexts: square M2L) */
-    SFMM_KERNELS_GENERIC = 3 /* one workgroup per translation, any orders <= 86 */
+    SFMM_KERNELS_GENERIC = 3 /* one workgroup per translation, any orders <= 86 (AUTO: several waves per 16
+                                translations for orders 25 to 48) */
 };
 
 /* Error codes (mirror the reference's exception types). */

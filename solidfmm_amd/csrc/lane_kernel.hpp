@@ -20,7 +20,7 @@
 // and the folded swap blocks are half zeros, which a VALU contraction skips
 // and an MFMA tile cannot.
 //
-// Two variants per (op, PI, PO):
+// Three variants per (op, PI, PO):
 //   RT = false  every item of the launch has orders (PI, PO) exactly;
 //   RT = true   PI = PO = PB is a bound and each item brings its own
 //               p_in, p_out <= PB (mixed-order lists).  A missing source
@@ -29,9 +29,9 @@
 //               (the z-translation sums only over K < p_in); output degrees
 //               >= p_out are not stored.  Degrees above the largest order
 //               of the wave are skipped with wave-uniform branches, so a
-//               wave of equal orders does the work of its own orders.
-//               With SUMS, for lists whose targets repeat in long runs, a
-//               wave of few runs adds them through LDS (run_sums).
+//               wave of equal orders does the work of its own orders;
+//   SUMS        as RT, for lists whose targets repeat in long runs: a wave
+//               of few runs adds them through LDS (run_sums).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -294,8 +294,9 @@ __device__ __forceinline__ void segment_sum(const Segments &g, double (&re)[N + 
 // each over every fourth (second) lane of a run, and the run's block is
 // stored as whole lines.  `on`: this lane's run has degree N.  In order-8
 // interaction lists, with runs of up to 64 items, 864 shuffles a wave become
-// 232 LDS accesses, and M2L with its reduction goes from 100.5 to 71.3 us
-// (14^3 cells; order 10: 213 -> 145, order 12: 368 -> 232).
+// 232 LDS accesses, and M2L with its reduction goes from 100.5 to 70.4 us
+// (14^3 cells; order 10: 213 -> 145, order 12: 368 -> 232).  Of short runs it
+// is the slower way (long_runs, kFewRuns).
 template <int N, int ST>
 __device__ __forceinline__ void run_sums(const Segments &g, double *buf, double *D, const double (&re)[N + 1],
                                          const double (&im)[N + 1], bool on)

@@ -1,5 +1,5 @@
 // FP64 translation kernel of one wave per eight translations of any orders
-// up to a bound, for long lists of orders 8 to 24.
+// up to a bound, for long lists of orders 8 to 24 (M2L to 22).
 //
 //   forward, per input degree n:   scale, rotate by alpha, swap, rotate by
 //                                  beta, swap; the degree stays in registers
@@ -51,7 +51,8 @@
 namespace sfmm {
 namespace octet {
 
-// 16 bytes at 8-byte alignment: blocks may start at any coefficient
+// 16 bytes at 8-byte alignment: a piece may start at any coefficient of its
+// block
 typedef double dbl2 __attribute__((ext_vector_type(2), aligned(8)));
 
 inline constexpr int kItems = 8;  // translations per wave

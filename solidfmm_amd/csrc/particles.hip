@@ -313,7 +313,8 @@ __global__ void __launch_bounds__(64)
 
 // The walk over the coefficients of an order-P block: degrees m..P-1 of order
 // m, column by column, in groups of kGroup.  A step that starts a column
-// takes R_m^m and makes R_{m+1}^{m+1} = c (x + iy) R_m^m, c = 1/(2m+2); the others are R_n^m = z c R_{n-1}^m - |x|^2 f R_{n-2}^m with
+// takes R_m^m and makes R_{m+1}^{m+1} = c (x + iy) R_m^m, c = 1/(2m+2); the
+// others are R_n^m = z c R_{n-1}^m - |x|^2 f R_{n-2}^m with
 // f = 1/((n+m)(n-m)) and c = (2n-1) f (c = 1 at n = m+1, where R_{n-2}^m is
 // zero).  Past the last coefficient c = f = 0 and nm has n = P.
 struct Step {

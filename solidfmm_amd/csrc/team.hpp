@@ -26,8 +26,8 @@
 // instruction cache).  A lone group is bound by its chain of degrees, which
 // the waves walk side by side; a full chip by the FP64 pipe that matrix and
 // vector instructions share.  M2L of order 32: 2,003 translations 577 us on
-// the one-workgroup-per-translation kernel, 37 us here; 30,000 7.7 ms and
-// 0.37 ms (97 us would be the FP64 pipe's time at its measured 47 TFLOP/s).
+// the one-workgroup-per-translation kernel, 38 us here; 30,000 7.7 ms and
+// 0.34 ms (97 us would be the FP64 pipe's time at its measured 47 TFLOP/s).
 // Orders up to 24 come here on lists too short to fill the chip with
 // octet.hpp's groups (team_items): M2L of order 8, 500 translations took 8.8
 // us on lanes and 5.2 here.

@@ -1,11 +1,11 @@
 // Dispatch of the translation kernels: (op, kernel choice) -> launch.
 //
 // The kernels themselves live in lane_kernel.hpp (one lane per
-// translation), octet.hpp and team.hpp (8 or 16 translations per group on the FP64
-// matrix cores), team.hpp (up to 16 translations per workgroup, orders 25 to
-// 48), generic.hip (one workgroup per translation, any order) and,
-// for the reduced-precision modes, lane_prec.hpp, mfma_prec.hpp (FP32
-// matrix cores) and prec_generic.hip.
+// translation), octet.hpp (a wave per 8 translations on the FP64 matrix
+// cores) and team.hpp (several waves per 16, short lists and orders to 48),
+// generic.hip (one workgroup per translation, any order) and, for the
+// reduced-precision modes, lane_prec.hpp, mfma_prec.hpp (FP32 matrix cores)
+// and prec_generic.hip.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>

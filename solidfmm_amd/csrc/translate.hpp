@@ -17,7 +17,7 @@ namespace sfmm {
 //            eight translations (octet.hpp, long lists) or several waves per
 //            sixteen (team.hpp);
 //   generic  any orders up to 86, one workgroup per translation
-//            (generic.hip); orders 25 to 48 on the team kernels (team.hpp)
+//            (generic.hip); orders 25 to 48 run on the team kernels (team.hpp)
 //            unless the context asks for this family.
 // Lane and octet kernels are instantiated per order bound PB.  Lane kernels
 // take items of orders (PB, PB), their RT variants any p_in, p_out <= PB, as
@@ -104,8 +104,9 @@ inline constexpr uint32_t kPairsMin = 13, kPairsMax = 17;
 size_t team_items(int op, uint32_t pb);
 
 // Launches above kLaneAutoMax that stay on lanes: n items of distinct targets
-// (shared: whose list reads a source twice or more on average), and n of the `total` items of a plan of repeated targets that are `runs` runs
-// in lane waves.
+// (shared: whose list reads a source twice or more on average), and n of the
+// `total` items of a plan of repeated targets that are `runs` runs in lane
+// waves.
 bool lanes_ahead(int op, uint32_t pb, size_t n, bool shared);
 bool lanes_for_runs(int op, uint32_t pb, size_t n, size_t runs, size_t total);
 
