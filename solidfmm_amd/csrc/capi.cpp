@@ -1490,7 +1490,6 @@ int sfmm_cellset_create(sfmm_context *ctx, const sfmm_cell *cells, size_t n, siz
     *out = nullptr;
     if (n && !cells) return fail(ctx, SFMM_ERR_LOGIC, "solidfmm: null cell list");
     size_t extent = 0;
-    sfmm::CellCounts counts;
     const uint32_t dim = n ? std::max(cells[0].dim, 1u) : 1u;
     if (dim > uint32_t(sfmm::kMaxParticleDim))
         return fail(ctx, SFMM_ERR_LOGIC, "solidfmm: particle expansions of dimension 1..4 only");
@@ -1501,14 +1500,13 @@ int sfmm_cellset_create(sfmm_context *ctx, const sfmm_cell *cells, size_t n, siz
         if (uint64_t(c.first) + c.count > n_points) return fail(ctx, SFMM_ERR_LOGIC, "solidfmm: cell points out of range");
         if (std::max(c.dim, 1u) != dim) return fail(ctx, SFMM_ERR_LOGIC, "solidfmm: cells of one set must share dim");
         extent = std::max<size_t>(extent, c.offset + size_t(dim) * c.order * (c.order + 1));
-        counts.add(c);
     }
     sfmm_cellset *set = new (std::nothrow) sfmm_cellset;
     if (!set) return fail(ctx, SFMM_ERR_ALLOC, "solidfmm: out of host memory");
     set->ctx = ctx;
     set->n_points = n_points;
     set->pool_extent = extent;
-    set->counts = counts;
+    set->counts = sfmm::count_cells(cells, n, int(dim));
     set->dim = int(dim);
     hipError_t e = hipSetDevice(ctx->device);
     if (e == hipSuccess && n) {

@@ -39,7 +39,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <cmath>
 #include <cstdint>
 
 #include "../../include/solidfmm_gpu.h"
@@ -671,9 +670,9 @@ constexpr size_t kWavesP2M = 5632, kWavesL2P = 1792;
 constexpr size_t kStageBytes = 9 * 1024;
 
 // P2M takes a wave per cell where the cells have so few points that the walk
-// would mostly be for lanes without one: up to `few` points a cell (four times
-// that in the largest, a wave of its own in both kernels).  Where the kernel
-// per cell was no slower, in us against the walk's:
+// would mostly be for lanes without one: up to `few` and a half on average,
+// four times `few` in the largest, which a wave goes through by itself.  Where
+// the kernel per cell was no slower, in us against the walk's:
 //   orders to 10, a cell's coefficients one pass of a wave: up to 6 while the
 //   cells are in flight at once (30,000 points of order 8, one charge: 17 and
 //   22 at 4 a cell, 21 and 14 at 12), 4 of very few cells; of many cells 2 or
@@ -682,6 +681,9 @@ constexpr size_t kStageBytes = 9 * 1024;
 //   above: 2 of few cells; of many 3 or 4, with one charge 1 and from order 20
 //   on 2 to 4, as the staged blocks leave the walk fewer waves (200,000 points
 //   of order 24, one charge: 1126 and 1634 at 3 a cell, 997 and 821 at 6).
+// The walk takes every cell of a run to the largest order, so 2 are always few
+// in sets of several (1,000,000 points, a quarter of the cells of order 16,
+// the others of 5, one charge, 2 a cell: 1001 and 1721).
 bool per_cell_p2m(const CellCounts &c, int dim)
 {
     const uint32_t P = c.max_order;
@@ -694,37 +696,38 @@ bool per_cell_p2m(const CellCounts &c, int dim)
     } else if (c.cells < 1024) few = 2;
     else if (dim == 1) few = P >= 24 ? 4 : P >= 20 ? 2 : 1;
     else few = P >= 16 || dim == 4 ? 4 : 3;
-    return c.points <= few * c.cells && c.most <= 4 * few;
+    if (c.mixed) few = std::max(few, size_t(2));
+    return 2 * c.points <= (2 * few + 1) * c.cells && c.most <= 4 * few;
 }
 
 // L2P takes a wave per cell where cells fill their own chunks of 64 lanes so
-// well that the walk, whose runs share chunks, has few less to go through: one
-// of its chunks costs as much as 1 / (share + slope (P - 4)) of the kernel
-// per cell.  The cells must fill the chip as well, from `cells` times the
-// order on for cells of one chunk.  The lines are fitted to the times of both
-// kernels at orders 4 to 32, 1 to 1,000 points a cell and 2,000 to 1,000,000
-// points, where the chosen one is on average 0.4 % behind the faster.
-// 1,000,000 points of order 8, three charges, per cell and on the walk: 131
-// and 210 us at 64 points a cell, 311 and 164 at 24; of order 10, one charge,
-// 123 and 97 at 64.  Order 4 with all chunks in flight at once gains nothing
-// from the exchange through LDS with more than one charge (30,000 points, three
-// charges, 24 a cell: 8.8 and 10.9; 60,000 points, one charge, 12 a cell: 10.0
-// and 9.0).
+// well that the walk, whose runs share chunks, has few less to go through, or
+// where it would take cells of low orders to the run's largest.  A chunk's
+// work by its order is chunk_work in the kernel per cell and as much over
+// (share + slope (order - 4)) on the walk; CellCounts holds the sums of both.
+// The cells must fill the chip as well, from `cells` times the order on for
+// cells of one chunk.  The lines are fitted to the times of both kernels at
+// orders 4 to 32, 1 to 1,000 points a cell and 2,000 to 1,000,000 points,
+// where the chosen one is on average 0.4 % behind the faster, 0.7 % in sets of
+// two orders.  1,000,000 points of order 8, three charges, per cell and on the
+// walk: 131 and 210 us at 64 points a cell, 311 and 164 at 24; of order 10,
+// one charge, 123 and 97 at 64; a quarter of the cells of order 10, the
+// others of 3, three charges, 64 a cell on average, 191 and 313.
+struct Line {
+    double share, slope;
+    uint32_t cells;
+};
+constexpr Line kLine[kMaxParticleDim] = {{0.40, 0.15, 375}, {0.45, 0.06, 256}, {0.35, 0.08, 192}, {0.40, 0.03, 128}};
+double chunk_work(uint32_t order) { return double(order) * (order + 1) + 20.0; }
+
+// Order 4 with all chunks in flight at once gains nothing from the exchange
+// through LDS with more than one charge (30,000 points, three charges, 24 a
+// cell: 8.8 and 10.9; 60,000 points, one charge, 12 a cell: 10.0 and 9.0).
 bool per_cell_l2p(const CellCounts &c, int dim)
 {
-    struct Line {
-        double share, slope;
-        uint32_t cells;
-    };
-    constexpr Line kLine[kMaxParticleDim] = {{0.40, 0.15, 375}, {0.45, 0.06, 256}, {0.35, 0.08, 192}, {0.40, 0.03, 128}};
-    const Line &line = kLine[dim - 1];
-    const uint32_t P = c.max_order;
-    if (P <= 4 && dim > 1 && c.most <= 64 && c.cells <= 5120) return true;
-    const size_t run = run_length(c.cells, kWavesL2P), runs = (c.cells + run - 1) / run;
-    const double walk = double(runs) * std::ceil(double(c.quads) * double(run) / double(16 * c.cells));
+    if (c.max_order <= 4 && dim > 1 && c.most <= 64 && c.cells <= 5120) return true;
     const uint64_t deepest = c.most / 64 + (c.most % 64 != 0);
-    return walk >= (line.share + line.slope * (int(P) - 4)) * double(c.chunks) &&
-           c.chunks >= deepest * line.cells * P;
+    return c.walk >= c.single && c.chunks >= deepest * kLine[dim - 1].cells * c.max_order;
 }
 
 template <int D>
@@ -766,6 +769,36 @@ hipError_t l2p_d(const double *pts, const sfmm_cell *cells, const CellCounts &c,
 }
 
 }  // namespace
+
+CellCounts count_cells(const sfmm_cell *cells, size_t n, int dim)
+{
+    CellCounts c;
+    c.cells = n;
+    const Line &line = kLine[dim - 1];
+    const uint32_t run = run_length(n, kWavesL2P);
+    uint32_t some = 0;  // order of a cell with points
+    for (size_t first = 0; first < n; first += run) {
+        uint64_t quads = 0;
+        uint32_t order = 0;
+        for (size_t i = first; i < std::min(n, first + run); ++i) {
+            const sfmm_cell &cell = cells[i];
+            c.max_order = std::max(c.max_order, cell.order);
+            if (cell.count == 0) continue;
+            const uint32_t chunks = cell.count / 64 + (cell.count % 64 != 0);
+            c.most = std::max(c.most, cell.count);
+            c.points += cell.count;
+            c.chunks += chunks;
+            c.single += chunks * chunk_work(cell.order);
+            c.mixed = c.mixed || (some && some != cell.order);
+            some = cell.order;
+            quads += cell.count / 4 + (cell.count % 4 != 0);
+            order = std::max(order, cell.order);
+        }
+        c.walk += double((quads + 15) / 16) * chunk_work(order) /
+                  (line.share + line.slope * double(std::max(order, 4u) - 4));
+    }
+    return c;
+}
 
 hipError_t launch_p2m(const double *pts, const sfmm_cell *cells, const CellCounts &counts, double *pool, int dim,
                       hipStream_t stream)

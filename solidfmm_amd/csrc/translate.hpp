@@ -183,21 +183,16 @@ hipError_t launch_generic(int op, uint32_t pc, const sfmm_item *items, size_t n,
 // Particle-side operators over device-resident cells (particles.hip).
 // dim: values per point and blocks per cell, 1..kMaxParticleDim.
 inline constexpr int kMaxParticleDim = 4;
+// What the launches need to know of a set's cells.
 struct CellCounts {
     size_t cells = 0;
     uint32_t max_order = 0;
     uint32_t most = 0;                // points of the largest cell
-    uint64_t points = 0, quads = 0, chunks = 0;  // sums of count, ceil(count / 4), ceil(count / 64)
-    void add(const sfmm_cell &c)
-    {
-        ++cells;
-        max_order = c.order > max_order ? c.order : max_order;
-        most = c.count > most ? c.count : most;
-        points += c.count;
-        quads += c.count / 4 + (c.count % 4 != 0);
-        chunks += c.count / 64 + (c.count % 64 != 0);
-    }
+    uint64_t points = 0, chunks = 0;  // sums of count and ceil(count / 64)
+    bool mixed = false;               // cells of several orders
+    double walk = 0.0, single = 0.0;  // L2P's work by runs and by cells (particles.hip)
 };
+CellCounts count_cells(const sfmm_cell *cells, size_t n, int dim);
 hipError_t launch_p2m(const double *pts, const sfmm_cell *cells, const CellCounts &counts, double *pool, int dim,
                       hipStream_t stream);
 hipError_t launch_l2p(const double *pts, const sfmm_cell *cells, const CellCounts &counts, const double *pool,

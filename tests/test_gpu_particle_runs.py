@@ -89,36 +89,43 @@ def test_runs_of_cells(sfmm, n_cells, orders, D):
 # cell (4 and 5 at 512 cells, 6 and 7 above, 3 and 4 or 4 and 5 of higher
 # orders), a larger cell among them (24 and 25 points of 6 a cell on average),
 # 5120 and 5121 cells of order 4, the share of lanes with a point (26 and 27 of
-# 64), the cells (767 and 768), a cell of two chunks; and the orders' ends.
-@pytest.mark.parametrize("n_cells,count,largest,P,D", [
-    (512, 4, 4, 8, 1), (512, 5, 5, 8, 1), (513, 6, 6, 10, 2), (513, 7, 7, 10, 2), (600, 5, 24, 6, 1), (600, 5, 25, 6, 1),
-    (1024, 3, 3, 12, 2), (1024, 4, 4, 12, 2), (1100, 4, 4, 16, 3), (1100, 5, 5, 16, 3), (1100, 3, 3, 32, 1),
-    (17000, 2, 2, 8, 3), (17000, 1, 1, 1, 2), (5120, 9, 9, 4, 2), (5121, 9, 9, 4, 2), (768, 27, 27, 8, 4),
-    (768, 26, 26, 8, 4), (767, 27, 27, 8, 4), (1000, 64, 65, 8, 4), (3100, 40, 40, 5, 1)])
-def test_sides_of_the_lines(sfmm, n_cells, count, largest, P, D):
+# 64), the cells (767 and 768), a cell of two chunks, the orders' ends; and
+# cells of two orders, every fourth of the first.
+@pytest.mark.parametrize("n_cells,count,largest,orders,D", [
+    (512, 4, 4, [8], 1), (512, 5, 5, [8], 1), (513, 6, 6, [10], 2), (513, 7, 7, [10], 2), (600, 5, 24, [6], 1),
+    (600, 5, 25, [6], 1), (1024, 3, 3, [12], 2), (1024, 4, 4, [12], 2), (1100, 4, 4, [16], 3), (1100, 5, 5, [16], 3),
+    (1100, 3, 3, [32], 1), (17000, 2, 2, [8], 3), (17000, 1, 1, [1], 2), (5120, 9, 9, [4], 2), (5121, 9, 9, [4], 2),
+    (768, 27, 27, [8], 4), (768, 26, 26, [8], 4), (767, 27, 27, [8], 4), (1000, 64, 65, [8], 4), (3100, 40, 40, [5], 1),
+    (2000, 2, 2, [16, 5], 1), (2000, 3, 3, [16, 5], 1), (3100, 20, 20, [10, 3], 3), (6000, 8, 8, [10, 3], 3),
+    (3100, 64, 65, [24, 8], 4)])
+def test_sides_of_the_lines(sfmm, n_cells, count, largest, orders, D):
     orc = oracle.Oracle()
-    rng = np.random.default_rng(n_cells + 10 * count + P)
+    rng = np.random.default_rng(n_cells + 10 * count + orders[0])
+    order = np.where(np.arange(n_cells) % 4 == 0, orders[0], orders[-1])
     counts = np.full(n_cells, count)
     counts[n_cells // 2] = largest
-    B = P * (P + 1)
     cells = np.zeros(n_cells, dtype=sfmm.CELL_DTYPE)
     ctr = rng.uniform(-2, 2, (n_cells, 3))
     cells["x"], cells["y"], cells["z"] = ctr.T
-    cells["offset"] = np.arange(n_cells) * D * B
+    size = D * order * (order + 1)
+    cells["offset"] = np.cumsum(size) - size
     cells["first"] = np.cumsum(counts) - counts
-    cells["count"], cells["order"], cells["dim"] = counts, P, D
+    cells["count"], cells["order"], cells["dim"] = counts, order, D
     n = int(counts.sum())
     pts = np.concatenate([np.repeat(ctr, counts, axis=0) + rng.uniform(-0.5, 0.5, (n, 3)),
                           rng.uniform(-1, 1, (n, D))], axis=1)
-    pool0 = rng.standard_normal((n_cells, D, B))
-    cs = sfmm.CellSet(sfmm.Context(P), cells, n)
-    pool, phi, grad = dev(pool0.reshape(-1)), dev(np.zeros((n, D))), dev(np.zeros((n, D, 3)))
+    pool0 = rng.standard_normal(int(size.sum()))
+    cs = sfmm.CellSet(sfmm.Context(max(orders)), cells, n)
+    pool, phi, grad = dev(pool0), dev(np.zeros((n, D))), dev(np.zeros((n, D, 3)))
     cs.l2p(dev(pts), pool, phi, grad)
     cs.p2m(dev(pts), pool)
     torch.cuda.synchronize()
-    got, phi, grad = pool.cpu().numpy().reshape(n_cells, D, B), phi.cpu().numpy(), grad.cpu().numpy()
+    got, phi, grad = pool.cpu().numpy(), phi.cpu().numpy(), grad.cpu().numpy()
     for s in [0, 1, 7, n_cells // 2, n_cells - 2, n_cells - 1]:
-        want = pool0[s].copy()
+        P = int(order[s])
+        block = slice(int(cells["offset"][s]), int(cells["offset"][s] + size[s]))
+        blocks = pool0[block].reshape(D, -1)
+        want = blocks.copy()
         at = slice(int(cells["first"][s]), int(cells["first"][s]) + int(counts[s]))
         ph, gr = np.zeros((counts[s], D)), np.zeros((counts[s], D, 3))
         for i, p in enumerate(pts[at]):
@@ -126,9 +133,9 @@ def test_sides_of_the_lines(sfmm, n_cells, count, largest, P, D):
             R, dR = orc.harmonic("R", P, *d), orc.harmonic("dR", P, *d).reshape(3, -1)
             for k in range(D):
                 want[k] += p[3 + k] * R
-                b = np.ascontiguousarray(pool0[s, k])
+                b = np.ascontiguousarray(blocks[k])
                 ph[i, k] = orc.dot(b, P, R, P)
                 gr[i, k] = [orc.dot(b, P, np.ascontiguousarray(g), P) for g in dR]
-        assert np.abs(got[s] - want).max() <= 1e-13 * max(np.abs(want).max(), 1), s
+        assert np.abs(got[block] - want.reshape(-1)).max() <= 1e-13 * max(np.abs(want).max(), 1), s
         assert np.abs(phi[at] - ph).max() <= 1e-12 * np.abs(ph).max(), s
         assert np.abs(grad[at] - gr).max() <= 1e-12 * max(np.abs(gr).max(), 1e-300), s
